@@ -36,6 +36,7 @@ HIP_SOURCES = (
     "gguf_moe.hip",
     "gguf_moe_mfma.hip",
     "gguf_moe_router.hip",
+    "gguf_moe_gemm.hip",
 )
 
 ARCH = "gfx950"

@@ -177,12 +177,21 @@ hipError_t launch_moe_q40_mfma(const uint8_t *gate, const uint8_t *up, const uin
                                const float *x, const int32_t *ids, const float *wts, int T, int top_k, float *out,
                                uint8_t *ws, hipStream_t stream);
 
-// Pieces of the MoE pipeline shared by its two implementations (gguf_moe.hip,
-// gguf_moe_mfma.hip): routing (meta layout of moe_layout; tiles0 / tiles1 =
-// work items per expert and route group of the matrix-core passes) and the
-// route-order combine.
-hipError_t launch_moe_route(const int32_t *ids, const float *wts, int P, int E, int tiles0,
-                            int tiles1, int32_t *meta, hipStream_t stream);
+// K-quant experts, many routes each, as grouped GEMMs (gguf_moe_gemm.hip):
+// gate / up of one K-quant type, down of any, hidden and inter multiples of
+// 256, weights 2-byte and x 16-byte aligned.
+bool moe_gemm_supported(int gate_type, int up_type, int down_type, int E, int H, int I, int T, int top_k,
+                        const uint8_t *gate, const uint8_t *up, const uint8_t *down, const float *x);
+hipError_t launch_moe_gemm(int gate_type, int down_type, const uint8_t *gate, const uint8_t *up, const uint8_t *down,
+                           int E, int H, int I, const float *x, const int32_t *ids, const float *wts, int T,
+                           int top_k, float *out, uint8_t *ws, hipStream_t stream);
+
+// Pieces of the MoE pipeline shared by its implementations (gguf_moe.hip,
+// gguf_moe_mfma.hip, gguf_moe_gemm.hip): routing (meta layout of moe_layout;
+// group > 0: also the grouped GEMM's items of at most `group` routes) and
+// the route-order combine.
+hipError_t launch_moe_route(const int32_t *ids, const float *wts, int P, int E, int group, int32_t *meta,
+                            int2 *items, hipStream_t stream);
 hipError_t launch_moe_combine(const int32_t *ids, const float *wts, const float *ypair, int T,
                               int top_k, int H, int E, float *out, hipStream_t stream);
 // MoE router (gguf_moe_router.hip): logits [T, E] -> ids / wts [T, K] with

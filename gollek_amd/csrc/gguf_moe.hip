@@ -29,7 +29,8 @@
 // in LDS), all-Q4_K layers up to hidden 4096 on the v_dot4 kernels
 // (moe_expert_kernel, x and h as integer digit planes, gguf_dot4.hpp), and
 // anything else on moe_generic_expert_kernel (byte loads, any alignment).
-// launch_moe sends the shapes the matrix-core passes take there first
+// launch_moe sends K-quant layers with enough routes per expert to the grouped
+// GEMM (gguf_moe_gemm.hip) and the shapes the matrix-core passes take there
 // (more than 2048 routes as token slices of at most 2048 / top_k tokens).
 #include "gguf_block_dot.hpp"
 #include "gguf_dot4.hpp"
@@ -46,8 +47,7 @@ size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 }  // namespace
 
 // meta (int32): counts[E] | offsets[E+1] | pairs[P] | used[E] | nused |
-// items0[E+1] | items1[E+1] (work-item offsets of the used experts for the
-// gate/up and down passes of the matrix-core kernels)
+// nitems (and 2 E + 1 not used)
 MoeLayout moe_layout(int64_t tokens, int64_t top_k, int64_t hidden, int64_t inter,
                      int64_t experts) {
     MoeLayout L;
@@ -66,96 +66,109 @@ MoeLayout moe_layout(int64_t tokens, int64_t top_k, int64_t hidden, int64_t inte
 
 // Routing on one workgroup: per-expert counts of the valid routes (expert id
 // in range, weight != 0; MFP:222), their offsets, the route list stably
-// sorted by expert, the used experts in expert order, and per used expert
-// u the work-item offsets items0/items1 = prefix of tiles * ceil(count / 4)
-// for the two expert passes.  Wave 0 scans in chunks of 64 with DPP-free
+// sorted by expert, the used experts in expert order, and (group > 0) the
+// items of the grouped GEMM, (expert, first route in that order) for every
+// `group` routes of an expert.  Wave 0 scans in chunks of 64 with DPP-free
 // shuffles; the stable scatter ranks equal keys within a chunk by ballots.
-__global__ __launch_bounds__(256) void moe_route_kernel(const int32_t *__restrict__ ids,
-                                                        const float *__restrict__ wts, int P,
-                                                        int E, int tiles0, int tiles1,
-                                                        int32_t *__restrict__ meta, int keys_in_lds) {
-    extern __shared__ int32_t sh[];  // cnt[E], run[E], then (keys_in_lds) key[P]
-    int32_t *cnt = sh, *run = sh + E, *keys = sh + 2 * E;
+// The routes are cut into `chunks` runs, one a wave (1: all of them in wave
+// 0's scatter): each counts its own keys, so the scatters run side by side
+// (2048 routes: 23 us in one wave, 6.6 us in 16).
+constexpr int kRouteThreads = 1024;
+__global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const int32_t *__restrict__ ids,
+                                                                  const float *__restrict__ wts, int P, int E,
+                                                                  int group, int chunks, int32_t *__restrict__ meta,
+                                                                  int2 *__restrict__ items, int keys_in_lds) {
+    extern __shared__ int32_t sh[];  // cnt[E], run[chunks][E], then (keys_in_lds) key[P]
+    int32_t *cnt = sh, *run = sh + E, *keys = run + chunks * E;
     int32_t *counts = meta, *offsets = meta + E, *pairs = meta + 2 * E + 1;
     int32_t *used = pairs + P, *nused = used + E;
-    int32_t *items0 = nused + 1, *items1 = items0 + E + 1;
-    const int lane = threadIdx.x & 63;
-    for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
+    int32_t *nitems = nused + 1;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int per = ((P + chunks - 1) / chunks + 63) / 64 * 64;  // routes of a chunk
+    for (int i = tid; i < chunks * E; i += kRouteThreads) run[i] = 0;
     __syncthreads();
-    for (int p = threadIdx.x; p < P; p += blockDim.x) {
+    for (int p = tid; p < P; p += kRouteThreads) {
         const int e = ids[p];
         const bool valid = e >= 0 && e < E && wts[p] != 0.0f;
-        if (valid) atomicAdd(&cnt[e], 1);  // LDS atomic
+        if (valid) atomicAdd(&run[p / per * E + e], 1);  // LDS atomic
         if (keys_in_lds) keys[p] = valid ? e : -1;
     }
     __syncthreads();
-    if (threadIdx.x < 64) {
-        const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-        int carry = 0, ucount = 0, it0 = 0, it1 = 0;
+    for (int e = tid; e < E; e += kRouteThreads) {
+        int c = 0;
+        for (int k = 0; k < chunks; k++) {
+            const int n = run[k * E + e];
+            run[k * E + e] = c;
+            c += n;
+        }
+        cnt[e] = c;
+    }
+    __syncthreads();
+    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    if (tid < 64) {
+        int carry = 0, ucount = 0, icarry = 0;
         for (int base = 0; base < E; base += 64) {
             const int e = base + lane;
             const int c = e < E ? cnt[e] : 0;
-            const int groups = (c + 3) / 4;
-            int a = c, b0 = tiles0 * groups, b1 = tiles1 * groups;
+            const int groups = group > 0 ? (c + group - 1) / group : 0;
+            int a = c, b = groups;
             // inclusive scans over the 64 lanes
             for (int d = 1; d < 64; d <<= 1) {
-                const int ta = __shfl_up(a, d, 64), tb0 = __shfl_up(b0, d, 64), tb1 = __shfl_up(b1, d, 64);
+                const int ta = __shfl_up(a, d, 64), tb = __shfl_up(b, d, 64);
                 if (lane >= d) {
                     a += ta;
-                    b0 += tb0;
-                    b1 += tb1;
+                    b += tb;
                 }
             }
             const uint64_t ub = __ballot(c > 0);
             if (e < E) {
                 offsets[e] = carry + a - c;
                 counts[e] = c;
-                run[e] = carry + a - c;
+                cnt[e] = carry + a - c;
             }
-            if (c > 0) {
-                const int u = ucount + __popcll(ub & below);
-                used[u] = e;
-                items0[u] = it0 + b0 - tiles0 * groups;
-                items1[u] = it1 + b1 - tiles1 * groups;
-            }
+            if (c > 0) used[ucount + __popcll(ub & below)] = e;
+            for (int i = 0; i < groups; i++) items[icarry + b - groups + i] = make_int2(e, carry + a - c + group * i);
             carry += __shfl(a, 63, 64);
-            it0 += __shfl(b0, 63, 64);
-            it1 += __shfl(b1, 63, 64);
+            icarry += __shfl(b, 63, 64);
             ucount += __popcll(ub);
         }
         if (lane == 0) {
             offsets[E] = carry;
             *nused = ucount;
-            items0[ucount] = it0;
-            items1[ucount] = it1;
+            *nitems = icarry;
         }
-        // Stable scatter, 64 routes at a time in route order: a route's slot is
-        // its expert's running offset plus its rank among the chunk's equal keys.
-        int bits = 1;
-        while ((1 << bits) <= E) bits++;
-        for (int base = 0; base < P; base += 64) {
-            const int p = base + lane;
-            int key = -1;
-            if (p < P) {
-                if (keys_in_lds) {
-                    key = keys[p];
-                } else {
-                    const int e = ids[p];
-                    if (e >= 0 && e < E && wts[p] != 0.0f) key = e;
-                }
+    }
+    __syncthreads();
+    // Stable scatter, 64 routes at a time in route order: a route's slot is its
+    // expert's offset, plus the routes of it in earlier chunks and rounds, plus
+    // its rank among the round's equal keys.
+    if (wave >= chunks) return;
+    int32_t *const mine = run + wave * E;
+    int bits = 1;
+    while ((1 << bits) <= E) bits++;
+    const int end = (wave + 1) * per < P ? (wave + 1) * per : P;
+    for (int base = wave * per; base < end; base += 64) {
+        const int p = base + lane;
+        int key = -1;
+        if (p < end) {
+            if (keys_in_lds) {
+                key = keys[p];
+            } else {
+                const int e = ids[p];
+                if (e >= 0 && e < E && wts[p] != 0.0f) key = e;
             }
-            const uint32_t k1 = (uint32_t)(key + 1);
-            uint64_t same = __ballot(true);
-            for (int bt = 0; bt < bits; bt++) {
-                const uint64_t v = __ballot((k1 >> bt) & 1u);
-                same &= ((k1 >> bt) & 1u) ? v : ~v;
-            }
-            const int rank = __popcll(same & below);
-            const int r0 = key >= 0 ? run[key] : 0;  // read by all lanes before any update
-            if (key >= 0) pairs[r0 + rank] = p;
-            const bool last = (same >> lane) == 1ull;  // highest lane of its key
-            if (key >= 0 && last) run[key] = r0 + __popcll(same);
         }
+        const uint32_t k1 = (uint32_t)(key + 1);
+        uint64_t same = __ballot(true);
+        for (int bt = 0; bt < bits; bt++) {
+            const uint64_t v = __ballot((k1 >> bt) & 1u);
+            same &= ((k1 >> bt) & 1u) ? v : ~v;
+        }
+        const int rank = __popcll(same & below);
+        const int r0 = key >= 0 ? mine[key] : 0;  // read by all lanes before any update
+        if (key >= 0) pairs[cnt[key] + r0 + rank] = p;
+        const bool last = (same >> lane) == 1ull;  // highest lane of its key
+        if (key >= 0 && last) mine[key] = r0 + __popcll(same);
     }
 }
 
@@ -813,14 +826,17 @@ hipError_t launch_expert(int nsb, const uint8_t *w0, const uint8_t *w1, int64_t 
 
 }  // namespace
 
-hipError_t launch_moe_route(const int32_t *ids, const float *wts, int P, int E, int tiles0,
-                            int tiles1, int32_t *meta, hipStream_t stream) {
-    // The routes' keys stay in LDS for the scatter when they fit the default
-    // 64 KB (the scatter otherwise reloads them, one round trip per 64).
-    const size_t base = 2 * (size_t)E * sizeof(int32_t);
+hipError_t launch_moe_route(const int32_t *ids, const float *wts, int P, int E, int group,
+                            int32_t *meta, int2 *items, hipStream_t stream) {
+    // 16 chunks while their counters fit 32 KB, and the routes' keys in LDS for
+    // the scatter while everything fits the default 64 KB (it otherwise reloads
+    // them, one round trip per 64).
+    const int chunks = 16 * (size_t)E * sizeof(int32_t) <= 32768 ? 16 : 1;
+    const size_t base = (size_t)(1 + chunks) * (size_t)E * sizeof(int32_t);
     const int keys_in_lds = base + (size_t)P * sizeof(int32_t) <= 65536 ? 1 : 0;
-    hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(256), base + (keys_in_lds ? (size_t)P * sizeof(int32_t) : 0),
-                       stream, ids, wts, P, E, tiles0, tiles1, meta, keys_in_lds);
+    hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(kRouteThreads),
+                       base + (keys_in_lds ? (size_t)P * sizeof(int32_t) : 0), stream, ids, wts, P, E, group, chunks,
+                       meta, items, keys_in_lds);
     return hipGetLastError();
 }
 
@@ -873,7 +889,7 @@ hipError_t launch_moe_generic(int gate_type, int up_type, int down_type, const u
     const MoeLayout L = moe_layout(T, top_k, H, I, E);
     const int P = T * top_k;
     int32_t *meta = reinterpret_cast<int32_t *>(ws + L.meta);
-    hipError_t err = launch_moe_route(ids, wts, P, E, 0, 0, meta, stream);
+    hipError_t err = launch_moe_route(ids, wts, P, E, 0, meta, nullptr, stream);
     if (err != hipSuccess) return err;
     float *h = reinterpret_cast<float *>(ws + L.h);
     float *ypair = reinterpret_cast<float *>(ws + L.ypair);
@@ -957,6 +973,18 @@ hipError_t launch_moe_generic(int gate_type, int up_type, int down_type, const u
     return launch_moe_combine(ids, wts, ypair, T, top_k, H, E, out, stream);
 }
 
+// Whether the grouped GEMM's launches (about 45 us with nothing to read) are
+// the faster way: against the two-launch matrix-core passes from three routes
+// per expert and 56 routes (128 experts x 768, hidden 2048, Q4_K: 2 routes per
+// expert 101 us there, 108 here; 4 routes 147 / 119; 16 routes 396 / 166.
+// 64 x 1024, 3 routes: 102 / 77 us; 8 x 1536, 32 routes in all: 38 / 46 us, 64
+// routes: 50 / 46), against the row kernels, which take other shapes, from one
+// (32 x 1280, hidden 2816, Q4_K: 112 / 58 us).
+static bool moe_gemm_chosen(bool tile_passes, int E, int T, int top_k) {
+    const int64_t P = (int64_t)T * top_k;
+    return tile_passes ? P >= 3 * (int64_t)E && P >= 56 : P >= E;
+}
+
 hipError_t launch_moe(int gate_type, int up_type, int down_type, const uint8_t *gate, const uint8_t *up,
                       const uint8_t *down, int64_t gate_row_bytes, int64_t up_row_bytes,
                       int64_t down_row_bytes, int E, int H, int I, const float *x, const int32_t *ids,
@@ -983,9 +1011,15 @@ hipError_t launch_moe(int gate_type, int up_type, int down_type, const uint8_t *
         }
         return hipSuccess;
     }
-    // Q4_K or Q5_K gate / up with the down types the matrix-core passes take.
-    if (aligned && gate_type == up_type && tuning().moe_variant != 1 &&
-        moe_kq_mfma_supported(gate_type, down_type, E, H, I, T, top_k, x))
+    // K-quant experts with enough routes each: grouped GEMMs.  Otherwise
+    // Q4_K, Q5_K or Q6_K gate / up with the down types the matrix-core passes
+    // take.
+    const bool tile_passes = aligned && gate_type == up_type && tuning().moe_variant != 1 &&
+                             moe_kq_mfma_supported(gate_type, down_type, E, H, I, T, top_k, x);
+    if (tuning().moe_variant != 1 && moe_gemm_chosen(tile_passes, E, T, top_k) &&
+        moe_gemm_supported(gate_type, up_type, down_type, E, H, I, T, top_k, gate, up, down, x))
+        return launch_moe_gemm(gate_type, down_type, gate, up, down, E, H, I, x, ids, wts, T, top_k, out, ws, stream);
+    if (tile_passes)
         return launch_moe_kq_mfma(gate_type, down_type, gate, up, down, E, H, I, x, ids, wts, T, top_k, out, ws,
                                   stream);
     // All Q4_0 (hidden up to 2048): the matrix-core passes with Q4_0 rows.
@@ -1007,7 +1041,7 @@ hipError_t launch_moe_q4k_dot4(const uint8_t *gate, const uint8_t *up, const uin
     const MoeLayout L = moe_layout(T, top_k, H, I, E);
     const int P = T * top_k;
     int32_t *meta = reinterpret_cast<int32_t *>(ws + L.meta);
-    hipError_t rerr = launch_moe_route(ids, wts, P, E, 0, 0, meta, stream);
+    hipError_t rerr = launch_moe_route(ids, wts, P, E, 0, meta, nullptr, stream);
     if (rerr != hipSuccess) return rerr;
     hipLaunchKernelGGL(moe_digits_kernel, dim3(T), dim3(256), 0, stream, x, H, (int64_t)H,
                        ws + L.xdig, (int64_t)L.xdig_stride);

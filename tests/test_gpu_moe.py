@@ -193,6 +193,38 @@ def test_moe_prefill_token_slices(gt, dt, E, H, I, T, k):
         t.close()
 
 
+# The grouped GEMM (gguf_moe_gemm.hip: from three routes per expert and 56
+# routes): experts with c routes around its 16- and 32-row tiles beside one with
+# every token, an unused one, a route with an id out of range and one of weight
+# 0; items of 16 routes (E = 16) and 32 (E = 4); odd superblock counts, all type
+# pairs.  Norm-wise bound: the digits of x and h keep 2^-23, a row's sums take
+# at most 12 superblock additions of 2^-24 each whose terms (d P and dmin PM)
+# are up to 8 times the result: 12 * 8 * 2^-24 = 5.7e-6 a pass, two passes.
+@pytest.mark.parametrize("gt,dt,E,H,I,c", [
+    (syn.Q4_K, syn.Q4_K, 4, 256, 256, 1), (syn.Q4_K, syn.Q6_K, 16, 768, 512, 15),
+    (syn.Q5_K, syn.Q6_K, 4, 512, 256, 16), (syn.Q5_K, syn.Q5_K, 16, 256, 768, 17),
+    (syn.Q6_K, syn.Q4_K, 4, 1280, 256, 31), (syn.Q4_K, syn.Q5_K, 4, 512, 1280, 32),
+    (syn.Q6_K, syn.Q6_K, 4, 768, 768, 33), (syn.Q4_K, syn.Q4_K, 16, 3072, 512, 39)])
+def test_moe_grouped_gemm(gt, dt, E, H, I, c):
+    print(f"[gpu] moe gemm gate={gt} down={dt} E={E} H={H} I={I} c={c}", flush=True)
+    gate, up, down, tg, tu, td = _experts(E, H, I, seed=E + H + c, down_type=dt, gate_type=gt)
+    T, k = 40, 2
+    _, w = syn.moe_routing(T, E, k, seed=51)
+    ids = np.zeros((T, k), np.int32)
+    ids[c:, 0] = 2
+    ids[:, 1] = 1
+    ids[T - 1, 0] = E
+    w[T - 2, 1] = 0.0
+    x = syn.activation(T * H, seed=52).reshape(T, H)
+    out = ops.moe_grouped(tg, tu, td, E, x, ids, w)
+    ref = o.moe_reference_q4k(gate, up, down, E, x, ids, w, down_type=dt, gate_type=gt)
+    err = np.linalg.norm(out.astype(np.float64) - ref) / np.linalg.norm(ref)
+    print(f"[gpu] moe gemm err={err:.3e} rel_err={o.rel_err(out, ref):.3e}", flush=True)
+    assert err <= 2 * 5.7e-6 and o.rel_err(out, ref) <= MOE_TOL
+    for t in (tg, tu, td):
+        t.close()
+
+
 @pytest.fixture
 def moe_variant():
     def set_variant(v):
