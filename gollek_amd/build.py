@@ -37,6 +37,7 @@ HIP_SOURCES = (
     "gguf_moe_mfma.hip",
     "gguf_moe_router.hip",
     "gguf_moe_gemm.hip",
+    "gguf_kq_gemm.hip",
 )
 
 ARCH = "gfx950"

@@ -30,6 +30,7 @@
 #include "gguf_block_dot.hpp"
 #include "gguf_blocks.hpp"
 #include "gguf_dot4.hpp"
+#include "gguf_gemm_plan.hpp"
 #include "gguf_kernels.hpp"
 
 namespace gollek {
@@ -710,13 +711,22 @@ hipError_t launch_tiled(const uint8_t *w, int64_t row_bytes, const uint16_t *x, 
 
 size_t gemm_workspace_bytes(int type_id, int M, int N, int K) {
     if (type_id == kQ8_0 && M <= 32) return 0;  // the skinny kernel
+    if (type_id == kQ4_K || type_id == kQ5_K || type_id == kQ6_K) return kq_gemm_workspace_bytes(type_id, M, N, K);
     return gemm_tile_workspace_bytes(type_id, M, N, K);
 }
 
-// The need peaks at multiples of the 128-row tile and is zero once the tiles
-// cover the CUs; the splits keep (S - 1) tiles' partials per tile, below
-// cu_count 128 x 128 floats (16 MiB on 256 CUs).
+// Q8_0, Q4_0: the need peaks at multiples of the 128-row tile and is zero once
+// the tiles cover the CUs; the splits keep (S - 1) tiles' partials per tile,
+// below cu_count 128 x 128 floats (16 MiB on 256 CUs).  K-quants: the plans'
+// cap, or 7 partials of the largest M that splits.
 size_t gemm_workspace_max_bytes(int type_id, int N, int K) {
+    if (type_id == kQ4_K || type_id == kQ5_K || type_id == kQ6_K) {
+        int64_t m = 0;
+        for (int mt = 1; mt <= 64; mt++)
+            if (gemm_may_split(type_id, 128 * mt, N, K)) m = 128 * mt;
+        const size_t need = (size_t)7 * m * N * sizeof(float);
+        return need < kGemmMaxSplitBytes ? need : kGemmMaxSplitBytes;
+    }
     size_t most = 0;
     for (int mt = 1; mt <= 64; mt++) {
         const size_t b = gemm_workspace_bytes(type_id, 128 * mt, N, K);
@@ -747,7 +757,10 @@ hipError_t launch_gemm_bf16(int type_id, const uint8_t *w, int64_t row_bytes, co
                                row_bytes, x, y, M, N, K);
         return hipGetLastError();
     }
-    // 128 x 128 tiles for Q8_0, Q4_0 and Q4_K (K a multiple of 256).
+    // K-quants: codes widened in registers, fp16 matrix cores.
+    if (kq_gemm_supported(type_id, row_bytes, N, K, w, x))
+        return launch_kq_gemm(type_id, w, row_bytes, x, y, M, N, K, stream, workspace, workspace_bytes);
+    // 128 x 128 tiles for Q8_0 and Q4_0 (K a multiple of 256).
     if (gemm_tile_supported(type_id, row_bytes, M, N, K, w, x, y))
         return launch_gemm_tile(type_id, w, row_bytes, x, y, M, N, K, stream, workspace, workspace_bytes);
     // Other shapes and alignments.

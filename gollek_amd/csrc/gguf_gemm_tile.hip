@@ -1,5 +1,5 @@
 // gguf_gemm_tile.hip -- small-M GEMM (prefill / batched decode) Y = X . W^T
-// for Q8_0, Q4_0 and Q4_K weights on gfx950 bf16 MFMA, fp32 accumulate.
+// for Q8_0 and Q4_0 weights on gfx950 bf16 MFMA, fp32 accumulate.
 //
 // Y[M, N] = X[M, K] . W[N, K]^T with X bf16 (row-major M x K) and W the GGUF
 // matrix (N rows of K columns), the Linear convention of
@@ -8,23 +8,12 @@
 // GEMM: its prefill runs M independent raw mat-vecs per weight
 // (RT/GgufTensorOps.java:666-674; RT/ = runner/gguf/gollek-gguf-core/src/
 // main/java/tech/kayys/gollek/gguf/runtime/), each summing per block
-// d * sum(q * x) (RT/GgufQ8RawDot.java:137-184, RT/GgufQ32RawDot.java:33-66)
-// or, for Q4_K, per 32-element sub-block fl(d*sc) * sum(q * x) - fl(dmin*m)
-// * sum(x) (RT/GgufQ4RawDot.java:331-674).
+// d * sum(q * x) (RT/GgufQ8RawDot.java:137-184, RT/GgufQ32RawDot.java:33-66).
 //
-// Exactness.  Each v_mfma_f32_16x16x32_bf16 contracts one 32-element block
-// (or Q4_K sub-block) of X with the block's integer codes, which bf16 holds
-// exactly (Q8_0 q in [-127, 127], Q4_0 q - 8 in [-8, 7]; Q4_K as 128 + q,
-// q in [0, 15]); the block's fp32 scale is applied to that fp32 result in
-// one FMA per output, the reference's block structure.  The Q4_K min term
-// needs sum(x) over the sub-block per X row: one more MFMA per 16-row tile
-// with an all-ones B operand puts it in the same lanes as the products, and
-// a second FMA subtracts (dmin * m + 128 * d) times it, which also removes
-// the codes' offset of 128 (dmin * m is 0 when the min code is 0, so a
-// non-finite dmin stays out as in RT/GgufKQuantLayout.java:67-69).  The
-// offset makes the fp32 sums run at ~128 |x| instead of ~8 |x|: about 2^-17
-// of sum |x| of absolute error per sub-block, far inside the 1e-2 bar, and a
-// non-finite d gives NaN rather than +-inf.
+// Exactness.  Each v_mfma_f32_16x16x32_bf16 contracts one 32-element block of
+// X with the block's integer codes, which bf16 holds exactly (Q8_0 q in
+// [-127, 127], Q4_0 q - 8 in [-8, 7]); the block's fp32 scale is applied to
+// that fp32 result in one FMA per output, the reference's block structure.
 //
 // Tiling.  A workgroup owns a 128 x 128 tile of Y: 8 compute waves and 2
 // loader waves.  K advances in stages of 64 columns (two blocks).  Compute
@@ -76,17 +65,6 @@ constexpr int kStagePitch = kTileN + 4;        // floats per row of the output s
 //   Q8_0: the row's two 34-byte blocks (68 bytes; 5 chunks, the last 12
 //         bytes belong to the next stage and are not used)
 //   Q4_0: two 18-byte blocks (36 bytes; 3 chunks, 12 unused)
-//   Q4_K: the superblock header (16 bytes: d, dmin, 12 scale bytes) and the
-//         32 quant bytes of the stage's chunk c (sub-blocks 2c, 2c + 1)
-//   Q5_K: the header, the superblock's 32 qh bytes (bits 2c, 2c + 1 are the
-//         chunk's fifth bits) and the chunk's 32 quant bytes (80 bytes)
-//   Q6_K: the chunk's half (h = c >> 1) of ql (64 bytes) and of qh (32)
-//         from 0 or 2 bytes before them (m: superblocks of odd index begin 2
-//         bytes past a dword), and 32 bytes holding the scales and d (bytes
-//         192 .. 209) from byte 192 (m = 0) or 178 (m = 2): 5 + 3 + 2 chunks
-//         (160 bytes).  Rows of an even superblock count end with an odd
-//         superblock, so no load runs past a row's end; an even superblock's
-//         last chunk reads 14 bytes of the next one.
 template <int T>
 struct RawW;
 template <>
@@ -97,19 +75,6 @@ template <>
 struct RawW<kQ4_0> {
     static constexpr int kChunks = 3, kStageBytes = 36, kSlots = 6;
 };
-template <>
-struct RawW<kQ4_K> {
-    static constexpr int kChunks = 3, kStageBytes = 0, kSlots = 6;  // 144 bytes per four stages
-};
-template <>
-struct RawW<kQ5_K> {
-    static constexpr int kChunks = 5, kStageBytes = 0, kSlots = 6;  // 176 bytes per four stages
-};
-template <>
-struct RawW<kQ6_K> {
-    static constexpr int kChunks = 10, kStageBytes = 0, kSlots = 4;  // 210 bytes per four stages
-};
-
 // Geometry of a 16 MT x 128 tile: MT row tiles of 16 rows of X.  Tiles of
 // fewer rows (small M) are load-latency bound and use the LDS they leave free
 // for a deeper ring, as deep as the loader waves' vmcnt waits can count.
@@ -126,7 +91,6 @@ struct TileGeom {
     static constexpr int kDeep = (160 * 1024 / kSlot) < (63 / kLoads + 2) ? (160 * 1024 / kSlot) : (63 / kLoads + 2);
     static constexpr int kSlots = MT == 8 ? RawW<T>::kSlots : (kDeep < 8 ? kDeep : 8);
     static constexpr int kRing = kSlots * kSlot;
-    static constexpr bool kMins = T == kQ4_K || T == kQ5_K;
     static_assert(kRing <= 160 * 1024, "LDS budget");
     static_assert(kLoads * (kSlots - 2) <= 63, "vmcnt range of the loader waits");
     static_assert(kRing >= 4 * MT * 2 * 1024 && kRing >= kTileM * kStagePitch * 4, "epilogue staging");
@@ -146,15 +110,6 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 __device__ __forceinline__ void s8x4_bf16(uint32_t w, uint32_t &a, uint32_t &b) {
     a = pack_bf16x2((float)(int)(int8_t)(w & 0xFFu), (float)(int)(int8_t)((w >> 8) & 0xFFu));
     b = pack_bf16x2((float)(int)(int8_t)((w >> 16) & 0xFFu), (float)(int)(int8_t)(w >> 24));
-}
-
-// Four 4-bit codes q (one per byte of w) -> two dwords of bf16 pairs
-// holding 128 + q exactly: the bf16 bit pattern 0x4300 | q is 128 + q (at
-// 128 a bf16 step is 1), so one byte permute per pair instead of two
-// conversions.
-__device__ __forceinline__ void q4x4_bf16_128(uint32_t w, uint32_t &a, uint32_t &b) {
-    a = __builtin_amdgcn_perm(0x43434343u, w, 0x04010400u);  // {w.b0, 0x43, w.b1, 0x43}
-    b = __builtin_amdgcn_perm(0x43434343u, w, 0x04030402u);  // {w.b2, 0x43, w.b3, 0x43}
 }
 
 // 16-byte buffer->LDS load (a plain __device__ function: the builtin used
@@ -194,20 +149,14 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b) {
 // follows, so that no use is scheduled before the data has arrived.
 //
 // One stage's operands of a wave: per column tile i (rows 16 apart: +RP
-// bytes) the raw code dwords (q0..q2 at b; Q4_K: q0, q1) and the scale dword
-// (at s; Q4_K: the 16-byte header), then A (MT row tiles of X, at a +
-// 2048 i), each read by its own statement in that order (volatile asm keeps
+// bytes) the raw code dwords (q0..q2 at b) and the scale dword (at s), then A
+// (MT row tiles of X, at a + 2048 i), each read by its own statement in that order (volatile asm keeps
 // the order).  LDS reads complete in order, so the raw codes can be widened
 // once ops_wait_raw returns while the A tiles still arrive, and row tile i
 // waits only for its own data (ops_wait_a).
 struct Ops {
     u32x4 a[8];
-    uint32_t q[2][3], sc[2];  // Q8_0, Q4_0
-    uint2 q2[2];              // Q4_K, Q5_K
-    u32x4 hd[2];              // Q4_K, Q5_K
-    uint2 qh[2];              // Q5_K
-    uint32_t l6[2][3], h6[2][3], d6[2];  // Q6_K: ql, qh dwords, d
-    uint32_t s6[2][2];                   // Q6_K: scale bytes
+    uint32_t q[2][3], sc[2];
 };
 template <int RP>
 __device__ __forceinline__ void ops_read_q32(uint32_t b, uint32_t s, Ops &o) {
@@ -223,61 +172,6 @@ __device__ __forceinline__ void ops_read_q32(uint32_t b, uint32_t s, Ops &o) {
         : "=&v"(o.q[0][0]), "=&v"(o.q[0][1]), "=&v"(o.q[0][2]), "=&v"(o.sc[0]), "=&v"(o.q[1][0]),
           "=&v"(o.q[1][1]), "=&v"(o.q[1][2]), "=&v"(o.sc[1])
         : "v"(b), "v"(s), "n"(RP), "n"(RP + 4), "n"(RP + 8)
-        : "memory");
-}
-template <int RP>
-__device__ __forceinline__ void ops_read_q4k(uint32_t b, uint32_t s, Ops &o) {
-    asm volatile(
-        "ds_read_b64 %0, %4\n\t"
-        "ds_read_b128 %1, %5\n\t"
-        "ds_read_b64 %2, %4 offset:%6\n\t"
-        "ds_read_b128 %3, %5 offset:%6"
-        : "=&v"(o.q2[0]), "=&v"(o.hd[0]), "=&v"(o.q2[1]), "=&v"(o.hd[1])
-        : "v"(b), "v"(s), "n"(RP)
-        : "memory");
-}
-// Q5_K: ops_read_q4k plus the lane's 8 qh bytes of each column tile (at h).
-template <int RP>
-__device__ __forceinline__ void ops_read_q5k(uint32_t b, uint32_t s, uint32_t h, Ops &o) {
-    asm volatile(
-        "ds_read_b64 %0, %6\n\t"
-        "ds_read_b64 %1, %8\n\t"
-        "ds_read_b128 %2, %7\n\t"
-        "ds_read_b64 %3, %6 offset:%9\n\t"
-        "ds_read_b64 %4, %8 offset:%9\n\t"
-        "ds_read_b128 %5, %7 offset:%9"
-        : "=&v"(o.q2[0]), "=&v"(o.qh[0]), "=&v"(o.hd[0]), "=&v"(o.q2[1]), "=&v"(o.qh[1]), "=&v"(o.hd[1])
-        : "v"(b), "v"(s), "v"(h), "n"(RP)
-        : "memory");
-}
-// Q6_K: per column tile the lane's 3 ql dwords (at l), 3 qh dwords (at h),
-// the 2 dwords of scale bytes from s and the dword holding d (at dd).
-template <int RP>
-__device__ __forceinline__ void ops_read_q6k(uint32_t l, uint32_t h, uint32_t s, uint32_t dd, Ops &o) {
-    asm volatile(
-        "ds_read_b32 %0, %18\n\t"
-        "ds_read_b32 %1, %18 offset:4\n\t"
-        "ds_read_b32 %2, %18 offset:8\n\t"
-        "ds_read_b32 %3, %19\n\t"
-        "ds_read_b32 %4, %19 offset:4\n\t"
-        "ds_read_b32 %5, %19 offset:8\n\t"
-        "ds_read_b32 %6, %20\n\t"
-        "ds_read_b32 %7, %20 offset:4\n\t"
-        "ds_read_b32 %8, %21\n\t"
-        "ds_read_b32 %9, %18 offset:%22\n\t"
-        "ds_read_b32 %10, %18 offset:%23\n\t"
-        "ds_read_b32 %11, %18 offset:%24\n\t"
-        "ds_read_b32 %12, %19 offset:%22\n\t"
-        "ds_read_b32 %13, %19 offset:%23\n\t"
-        "ds_read_b32 %14, %19 offset:%24\n\t"
-        "ds_read_b32 %15, %20 offset:%22\n\t"
-        "ds_read_b32 %16, %20 offset:%23\n\t"
-        "ds_read_b32 %17, %21 offset:%22"
-        : "=&v"(o.l6[0][0]), "=&v"(o.l6[0][1]), "=&v"(o.l6[0][2]), "=&v"(o.h6[0][0]), "=&v"(o.h6[0][1]),
-          "=&v"(o.h6[0][2]), "=&v"(o.s6[0][0]), "=&v"(o.s6[0][1]), "=&v"(o.d6[0]), "=&v"(o.l6[1][0]),
-          "=&v"(o.l6[1][1]), "=&v"(o.l6[1][2]), "=&v"(o.h6[1][0]), "=&v"(o.h6[1][1]), "=&v"(o.h6[1][2]),
-          "=&v"(o.s6[1][0]), "=&v"(o.s6[1][1]), "=&v"(o.d6[1])
-        : "v"(l), "v"(h), "v"(s), "v"(dd), "n"(RP), "n"(RP + 4), "n"(RP + 8)
         : "memory");
 }
 template <int I>
@@ -303,21 +197,9 @@ __device__ __forceinline__ void ops_read_as(uint32_t a, Ops &o) {
 // The raw dwords have arrived (the MT A reads may still be outstanding).
 template <int MT>
 __device__ __forceinline__ void ops_wait_raw(Ops &o) {
-    asm volatile("s_waitcnt lgkmcnt(%14)"
+    asm volatile("s_waitcnt lgkmcnt(%8)"
                  : "+v"(o.q[0][0]), "+v"(o.q[0][1]), "+v"(o.q[0][2]), "+v"(o.sc[0]), "+v"(o.q[1][0]),
-                   "+v"(o.q[1][1]), "+v"(o.q[1][2]), "+v"(o.sc[1]), "+v"(o.q2[0]), "+v"(o.q2[1]),
-                   "+v"(o.hd[0]), "+v"(o.hd[1]), "+v"(o.qh[0]), "+v"(o.qh[1])
-                 : "n"(MT)
-                 : "memory");
-}
-// Q6_K: the same wait for its raw dwords.
-template <int MT>
-__device__ __forceinline__ void ops_wait_raw6(Ops &o) {
-    asm volatile("s_waitcnt lgkmcnt(%18)"
-                 : "+v"(o.l6[0][0]), "+v"(o.l6[0][1]), "+v"(o.l6[0][2]), "+v"(o.h6[0][0]), "+v"(o.h6[0][1]),
-                   "+v"(o.h6[0][2]), "+v"(o.s6[0][0]), "+v"(o.s6[0][1]), "+v"(o.d6[0]), "+v"(o.l6[1][0]),
-                   "+v"(o.l6[1][1]), "+v"(o.l6[1][2]), "+v"(o.h6[1][0]), "+v"(o.h6[1][1]), "+v"(o.h6[1][2]),
-                   "+v"(o.s6[1][0]), "+v"(o.s6[1][1]), "+v"(o.d6[1])
+                   "+v"(o.q[1][1]), "+v"(o.q[1][2]), "+v"(o.sc[1])
                  : "n"(MT)
                  : "memory");
 }
@@ -385,12 +267,7 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
     // the end read as zeros.
     const int mrows = M - m0 < kTileM ? M - m0 : kTileM;
     const int nrows = N - n0 < kTileN ? N - n0 : kTileN;
-    // (Q6_K: none; its loads start up to 2 bytes before a superblock, so the
-    // offsets stay relative to the rows' first byte)
-    const int64_t w_split = T == kQ4_K   ? (int64_t)(s0 / 4) * 144
-                            : T == kQ5_K ? (int64_t)(s0 / 4) * kQ5KBlockBytes
-                            : T == kQ6_K ? 0
-                                         : (int64_t)s0 * R::kStageBytes;
+    const int64_t w_split = (int64_t)s0 * R::kStageBytes;
     const __amdgpu_buffer_rsrc_t xr = wave_buffer(
         reinterpret_cast<const uint8_t *>(X) + (int64_t)m0 * K * 2 + (int64_t)s0 * 128,
         (uint32_t)((int64_t)mrows * K * 2 - (int64_t)s0 * 128));
@@ -402,8 +279,7 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
     // at swizzled position p % 8, holding the row's column chunk
     // position ^ ((row >> 1) & 7).  W: instruction j moves lane-chunks q =
     // 64 j + lane (row q / kChunks, part q % kChunks) to LDS offset 16 q;
-    // loader l takes instructions l, l + 2, ...  Q4_K: part 0 is the header,
-    // parts 1 and 2 the quants at 16 + 32 c + 16 (part - 1).
+    // loader l takes instructions l, l + 2, ...
     const int ldr = wave - 8;
     auto issue = [&](int ls) {
         uint8_t *const xs = ring + (ls % NS) * G::kSlot;
@@ -420,22 +296,8 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
             const int j = ldr + 2 * i;
             const int q = 64 * j + lane;
             const int row = q / R::kChunks, part = q - row * R::kChunks;
-            uint32_t off = (uint32_t)row * (uint32_t)row_bytes + (uint32_t)(16 * part);
-            if constexpr (T == kQ4_K)
-                off += (uint32_t)(144 * (ls >> 2)) + (part != 0 ? (uint32_t)(32 * (ls & 3)) : 0u);
-            else if constexpr (T == kQ5_K)  // parts 0..2: header, qh; 3, 4: the chunk's quants at 48
-                off += (uint32_t)(kQ5KBlockBytes * (ls >> 2)) + (part >= 3 ? (uint32_t)(32 * (ls & 3)) : 0u);
-            else if constexpr (T == kQ6_K) {
-                // superblock sb from its dword at or before it (m = 2 (sb & 1)); parts
-                // 0..4: ql half h from 64 h, 5..7: qh half h from 128 + 32 h (both
-                // less m), 8, 9: from 192 (m = 0) or 178 (m = 2)
-                const int sb = (s0 >> 2) + (ls >> 2), h = (ls >> 1) & 1, m2 = sb & 1;
-                const int at = part < 5 ? 64 * h + 16 * part
-                               : part < 8 ? 128 + 32 * h + 16 * (part - 5)
-                                          : (m2 ? 180 : 192) + 16 * (part - 8);
-                off = (uint32_t)row * (uint32_t)row_bytes + (uint32_t)(210 * sb - 2 * (sb & 1) + at);
-            } else
-                off += (uint32_t)(R::kStageBytes * ls);
+            const uint32_t off =
+                (uint32_t)row * (uint32_t)row_bytes + (uint32_t)(16 * part) + (uint32_t)(R::kStageBytes * ls);
             dma16(wr, rs + 1024 * j, off);
         }
     };
@@ -459,48 +321,34 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
         qsh = kg ? 0u : 2u;
         soff = (uint32_t)(32 * kg);
         nsh = 16u * (uint32_t)kg;  // scale half
-    } else if constexpr (T == kQ4_0) {
+    } else {
         // 8 bytes of block kg at byte 2 + 18 kg + 8 (lk & 1); nibble lk >> 1; scale in dword 4 kg
         qoff = (uint32_t)(4 * (kg ? 5 + 2 * (lk & 1) : 2 * (lk & 1)));
         qsh = kg ? 0u : 2u;
         soff = (uint32_t)(16 * kg);
         nsh = 16u * (uint32_t)kg;
-    } else {
-        // quant bytes 8 lk .. 8 lk + 7 of the chunk at 16 + 8 lk (Q5_K: at
-        // 48 + 8 lk, its qh bytes 8 lk .. 8 lk + 7 at 16 + 8 lk); header at 0
-        qoff = (uint32_t)((T == kQ5_K ? 48 : 16) + 8 * lk);
-        qsh = 0u;
-        soff = 0u;
-        nsh = 0u;
     }
-    const uint32_t qhoff = (uint32_t)(16 + 8 * lk);       // Q5_K
-    const int nib = T == kQ4_0 ? 4 * (lk >> 1) : 4 * kg;  // nibble shift (Q4_0, Q4_K, Q5_K)
+    const int nib = 4 * (lk >> 1);  // nibble shift (Q4_0)
 
     f32x4 acc[MT][2];
 #pragma unroll
     for (int a = 0; a < MT; a++)
 #pragma unroll
         for (int b = 0; b < 2; b++) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
 
-    // Per stage: 2 MT MFMAs (MT row tiles x 2 column tiles; Q4_K: one more
-    // per row tile for the sums of x) and one FMA (Q4_K: two) per output.
+    // Per stage: 2 MT MFMAs (MT row tiles x 2 column tiles) and one FMA per
+    // output.
     // The FMAs of each MFMA are issued two MFMAs later, so that no FMA waits
     // for the MFMA it consumes.
     auto compute = [&](int ls) {
         const uint32_t so = (uint32_t)((ls % NS) * G::kSlot);
         Ops o;
-        if constexpr (T == kQ4_K)
-            ops_read_q4k<16 * G::kPitch>(wrow + so + qoff, wrow + so + soff, o);
-        else if constexpr (T == kQ5_K)
-            ops_read_q5k<16 * G::kPitch>(wrow + so + qoff, wrow + so + soff, wrow + so + qhoff, o);
-        else
-            ops_read_q32<16 * G::kPitch>(wrow + so + qoff, wrow + so + soff, o);
+        ops_read_q32<16 * G::kPitch>(wrow + so + qoff, wrow + so + soff, o);
         ops_read_as<MT>(xa + so, o);
         ops_wait_raw<MT>(o);
         bf16x8 B[2];
-        float d[2], dm[2];
-        // Column tile i's codes as bf16 (B operand) and its scale / min term.
+        float d[2];
+        // Column tile i's codes as bf16 (B operand) and its scale.
         auto widen = [&](int i) {
             uint32_t c[4];
             if constexpr (T == kQ8_0) {
@@ -509,46 +357,25 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
                 s8x4_bf16(w0, c[0], c[1]);
                 s8x4_bf16(w1, c[2], c[3]);
                 d[i] = half_bits_to_float_fast(o.sc[i] >> nsh);
-            } else if constexpr (T == kQ4_0) {
+            } else {
                 // q - 8 as a signed byte: ((nib + 0x78) ^ 0x80)
                 const uint32_t w0 = (__builtin_amdgcn_alignbyte(o.q[i][1], o.q[i][0], qsh) >> nib) & 0x0F0F0F0Fu;
                 const uint32_t w1 = (__builtin_amdgcn_alignbyte(o.q[i][2], o.q[i][1], qsh) >> nib) & 0x0F0F0F0Fu;
                 s8x4_bf16((w0 + 0x78787878u) ^ 0x80808080u, c[0], c[1]);
                 s8x4_bf16((w1 + 0x78787878u) ^ 0x80808080u, c[2], c[3]);
                 d[i] = half_bits_to_float_fast(o.sc[i] >> nsh);
-            } else {
-                // B holds 128 + q; the 128 sum(x) it adds comes off with the
-                // min term: d (P - 128 sx) - dmin m sx = d P - (dmin m + 128 d) sx.
-                // Q5_K: q's fifth bit is bit 2 c + kg of its qh byte (c = ls & 3).
-                uint32_t lo = (o.q2[i].x >> nib) & 0x0F0F0F0Fu, hi = (o.q2[i].y >> nib) & 0x0F0F0F0Fu;
-                if constexpr (T == kQ5_K) {
-                    const int hb = 2 * (ls & 3) + kg;
-                    lo |= ((o.qh[i].x >> hb) & 0x01010101u) << 4;
-                    hi |= ((o.qh[i].y >> hb) & 0x01010101u) << 4;
-                }
-                q4x4_bf16_128(lo, c[0], c[1]);
-                q4x4_bf16_128(hi, c[2], c[3]);
-                uint32_t scp, mnp;
-                q4k_pair_codes(o.hd[i].y, o.hd[i].z, o.hd[i].w, ls & 3, &scp, &mnp);
-                const uint32_t scj = (scp >> (8 * kg)) & 0xFFu, mj = (mnp >> (8 * kg)) & 0xFFu;
-                d[i] = half_bits_to_float_fast(o.hd[i].x & 0xFFFFu) * (float)scj;
-                dm[i] = fmaf(128.0f, d[i], mj == 0u ? 0.0f : half_bits_to_float_fast(o.hd[i].x >> 16) * (float)mj);
             }
             B[i] = __builtin_bit_cast(bf16x8, u32x4{c[0], c[1], c[2], c[3]});
         };
         // MFMA k = 0 .. 2 MT - 1 is (row tile k % MT, column tile k / MT):
         // column tile 1 is widened while column tile 0's first MFMAs run, and
         // the FMAs of MFMA k - 2 are issued with MFMA k, so that none waits
-        // for its MFMA.  Q4_K: the sums of x of row tile mt come with its
-        // column-0 MFMA.
-        f32x4 p[3], sx[MT];
+        // for its MFMA.
+        f32x4 p[3];
         auto fmas = [&](int k) {
             const int mt = k % MT, nt = k / MT;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                acc[mt][nt][r] = fmaf(d[nt], p[k % 3][r], acc[mt][nt][r]);
-                if constexpr (G::kMins) acc[mt][nt][r] = fmaf(-dm[nt], sx[mt][r], acc[mt][nt][r]);
-            }
+            for (int r = 0; r < 4; r++) acc[mt][nt][r] = fmaf(d[nt], p[k % 3][r], acc[mt][nt][r]);
         };
         widen(0);
 #pragma unroll
@@ -559,89 +386,9 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
                 if (k < MT) ops_wait_row<MT>(k, o);
                 const bf16x8 A = __builtin_bit_cast(bf16x8, o.a[mt]);
                 if (k == (MT < 2 ? MT : 2)) widen(1);
-                if constexpr (G::kMins)
-                    if (nt == 0) sx[mt] = mfma_bf16(A, ones);
                 p[k % 3] = mfma_bf16(A, B[nt]);
             }
             if (k >= 2) fmas(k - 2);
-        }
-    };
-
-    // Q6_K: a 32-column block holds two 16-element scale groups, so each
-    // MFMA takes one group's codes (B_lo: lanes of k groups 0, 1; B_hi: 2, 3;
-    // the other lanes zero) as 128 + q (q = ql nibble | qh bits << 4, 0..63),
-    // starting from C = -160 sum(x) over the same lanes (an MFMA against a
-    // constant -160 B), so its result is sum((q - 32) x) of the group; the
-    // FMA applies fl(d sc) of the group (exact: an 11-bit d times an 8-bit
-    // scale).  Per row tile two MFMAs for the starts and per column tile two
-    // more, two FMAs per output.
-    auto compute6 = [&](int ls) {
-        const uint32_t so = (uint32_t)((ls % NS) * G::kSlot);
-        const int c = ls & 3, m = 2 * (((s0 >> 2) + (ls >> 2)) & 1);
-        const uint32_t rb = wrow + so;  // this lane's W row: ql piece, qh piece at 80, tail at 128
-        Ops o;
-        ops_read_q6k<16 * G::kPitch>(rb + 32 * kg + 8 * lk, rb + 80 + 8 * lk, rb + 128 + 4 * c + 6 * m,
-                                     rb + 144 + 6 * m, o);
-        ops_read_as<MT>(xa + so, o);
-        ops_wait_raw6<MT>(o);
-        const int nib = 4 * (c & 1), hsh = 2 * (2 * (c & 1) + kg);
-        const bool lo_half = lk < 2;
-        const u32x4 zero = {0u, 0u, 0u, 0u};
-        const u32x4 m160 = {0xC320C320u, 0xC320C320u, 0xC320C320u, 0xC320C320u};  // bf16 -160
-        const bf16x8 m160lo = __builtin_bit_cast(bf16x8, lo_half ? m160 : zero);
-        const bf16x8 m160hi = __builtin_bit_cast(bf16x8, lo_half ? zero : m160);
-        bf16x8 Blo[2], Bhi[2];
-        float dlo[2], dhi[2];
-        auto widen6 = [&](int i) {
-            const uint32_t l0 = __builtin_amdgcn_alignbyte(o.l6[i][1], o.l6[i][0], m);
-            const uint32_t l1 = __builtin_amdgcn_alignbyte(o.l6[i][2], o.l6[i][1], m);
-            const uint32_t h0 = __builtin_amdgcn_alignbyte(o.h6[i][1], o.h6[i][0], m);
-            const uint32_t h1 = __builtin_amdgcn_alignbyte(o.h6[i][2], o.h6[i][1], m);
-            const uint32_t q0 = ((l0 >> nib) & 0x0F0F0F0Fu) | (((h0 >> hsh) & 0x03030303u) << 4);
-            const uint32_t q1 = ((l1 >> nib) & 0x0F0F0F0Fu) | (((h1 >> hsh) & 0x03030303u) << 4);
-            uint32_t cc[4];
-            q4x4_bf16_128(q0, cc[0], cc[1]);
-            q4x4_bf16_128(q1, cc[2], cc[3]);
-            const u32x4 v = {cc[0], cc[1], cc[2], cc[3]};
-            Blo[i] = __builtin_bit_cast(bf16x8, lo_half ? v : zero);
-            Bhi[i] = __builtin_bit_cast(bf16x8, lo_half ? zero : v);
-            // the row's scales of groups 2 kg, 2 kg + 1 of the chunk, and d
-            const uint64_t sw = (((uint64_t)o.s6[i][1] << 32) | o.s6[i][0]) >> (8 * (m + 2 * kg));
-            const float d = half_bits_to_float_fast(o.d6[i] >> (8 * m));
-            dlo[i] = d * (float)(int)(int8_t)(sw & 0xFFu);
-            dhi[i] = d * (float)(int)(int8_t)((sw >> 8) & 0xFFu);
-        };
-        f32x4 plo[3], phi[3];
-        // MFMA pair k = 0 .. 2 MT - 1 is (row tile k / 2, column tile k % 2):
-        // the -160 sum(x) starts depend on the row tile only, so the two
-        // column tiles of a row tile take the same ones (six MFMAs per row
-        // tile); both column tiles are widened before the first MFMA.
-        auto fmas6 = [&](int k) {
-            const int mt = k >> 1, nt = k & 1;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                acc[mt][nt][r] = fmaf(dlo[nt], plo[k % 3][r], acc[mt][nt][r]);
-                acc[mt][nt][r] = fmaf(dhi[nt], phi[k % 3][r], acc[mt][nt][r]);
-            }
-        };
-        widen6(0);
-        widen6(1);
-        f32x4 tlo, thi;
-#pragma unroll
-        for (int k = 0; k < 2 * MT + 2; k++) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (k < 2 * MT) {
-                const int mt = k >> 1, nt = k & 1;
-                const bf16x8 A = __builtin_bit_cast(bf16x8, o.a[mt]);
-                if (nt == 0) {
-                    ops_wait_row<MT>(mt, o);
-                    tlo = mfma_bf16(A, m160lo);
-                    thi = mfma_bf16(A, m160hi);
-                }
-                plo[k % 3] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, Blo[nt], tlo, 0, 0, 0);
-                phi[k % 3] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, Bhi[nt], thi, 0, 0, 0);
-            }
-            if (k >= 2) fmas6(k - 2);
         }
     };
 
@@ -666,10 +413,7 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
     } else {
         for (int s = 0; s < nst; s++) {
             compute_barrier();
-            if constexpr (T == kQ6_K)
-                compute6(s);
-            else
-                compute(s);
+            compute(s);
         }
     }
 
@@ -758,8 +502,8 @@ namespace {
 // that small M computes no padding rows.  Q8_0 up to M = 128 with so few
 // column tiles that 128-row tiles would split K eight ways takes 64-row
 // tiles split four ways instead: three partial tiles per output in place of
-// seven (M = 128, N = 4096: 18.7 against 19.7 us; the K-quant and Q4_0
-// tiles at N = 14336 measured slower with 64 rows).
+// seven (M = 128, N = 4096: 18.7 against 19.7 us; the Q4_0 tiles at N =
+// 14336 measured slower with 64 rows).
 int tile_mt(int type_id, int M, int N) {
     if (M <= 16) return 1;
     if (M <= 32) return 2;
@@ -772,8 +516,7 @@ int tile_splits(int type_id, int M, int N, int K, size_t workspace_bytes) {
     const int tm = 16 * tile_mt(type_id, M, N);
     const int tiles = (M + tm - 1) / tm * ((N + kTileN - 1) / kTileN);
     const int nst = K / 64;
-    // A split holds a whole number of four-stage rounds (and so of Q4_K
-    // superblocks).
+    // A split holds a whole number of four-stage rounds.
     int S = 1;
     while (S < 8 && tiles * 2 * S <= device_cus() && nst % (8 * S) == 0 &&
            (size_t)(2 * S - 1) * M * N * sizeof(float) <= workspace_bytes)
@@ -785,14 +528,15 @@ int tile_splits(int type_id, int M, int N, int K, size_t workspace_bytes) {
 
 bool gemm_tile_supported(int type_id, int64_t row_bytes, int M, int N, int K, const void *w,
                          const void *x, const void *y) {
-    if (type_id != kQ8_0 && type_id != kQ4_0 && type_id != kQ4_K && type_id != kQ5_K && type_id != kQ6_K)
-        return false;
+    if (type_id != kQ8_0 && type_id != kQ4_0) return false;
     if (M <= 0 || N <= 0 || K % 256 != 0) return false;
     if (((reinterpret_cast<uintptr_t>(w) | (uintptr_t)row_bytes) & 3u) != 0) return false;
     if ((reinterpret_cast<uintptr_t>(x) & 15u) != 0 || (reinterpret_cast<uintptr_t>(y) & 15u) != 0) return false;
     // 32-bit buffer offsets: a tile's rows of X and W
     return (int64_t)kTileMMax * K * 2 < ((int64_t)1 << 31) && (int64_t)kTileN * row_bytes < ((int64_t)1 << 31);
 }
+
+bool gemm_may_split(int type_id, int M, int N, int K) { return tile_splits(type_id, M, N, K, (size_t)-1) > 1; }
 
 size_t gemm_tile_workspace_bytes(int type_id, int M, int N, int K) {
     const int S = tile_splits(type_id, M, N, K, (size_t)-1);
@@ -831,24 +575,16 @@ hipError_t launch_gemm_tile(int type_id, const uint8_t *w, int64_t row_bytes, co
     case kQ4_0:
         GOLLEK_TILE_LAUNCH(kQ4_0);
         break;
-    case kQ4_K:
-        GOLLEK_TILE_LAUNCH(kQ4_K);
-        break;
-    case kQ5_K:
-        GOLLEK_TILE_LAUNCH(kQ5_K);
-        break;
-    case kQ6_K:
-        GOLLEK_TILE_LAUNCH(kQ6_K);
-        break;
     default:
         return hipErrorInvalidValue;
     }
 #undef GOLLEK_TILE_LAUNCH
-    if (S > 1) {
-        const int64_t mn = (int64_t)M * N;
-        hipLaunchKernelGGL(gemm_tile_reduce_kernel, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0,
-                           stream, part, S - 1, mn, y);
-    }
+    return S > 1 ? launch_gemm_reduce(part, S, (int64_t)M * N, y, stream) : hipGetLastError();
+}
+
+hipError_t launch_gemm_reduce(const float *part, int S, int64_t mn, float *y, hipStream_t stream) {
+    hipLaunchKernelGGL(gemm_tile_reduce_kernel, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, stream, part,
+                       S - 1, mn, y);
     return hipGetLastError();
 }
 

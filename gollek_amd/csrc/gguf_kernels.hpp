@@ -97,13 +97,13 @@ hipError_t launch_gemv_k56(int type_id, const uint8_t *w, int64_t row_bytes, int
                            const float *x, float *y, int64_t rows, hipStream_t stream);
 
 
-// Y[M, N] = X[M, K] (bf16 bits) . W[N, K]^T for Q8_0, Q4_0 or Q4_K W
-// (gguf_gemm.hip, gguf_gemm_tile.hip).  Shapes whose output tiles leave CUs
-// idle are split over K into partial tiles in `workspace` (device memory of
+// Y[M, N] = X[M, K] (bf16 bits) . W[N, K]^T (gguf_gemm.hip, gguf_gemm_tile.hip,
+// gguf_kq_gemm.hip).  Shapes whose output tiles leave CUs idle are split over
+// K into partial tiles in `workspace` (device memory of
 // gemm_workspace_bytes(type, M, N, K) bytes; with less they split less or
 // run unsplit) and added in split order.
 size_t gemm_workspace_bytes(int type_id, int M, int N, int K);
-// The largest gemm_workspace_bytes(type, M, N, K) over every M.
+// At least gemm_workspace_bytes(type, M, N, K) of every M.
 size_t gemm_workspace_max_bytes(int type_id, int N, int K);
 // prep / prep_rows: the weight's prepared column layout (M <= 4 reads it
 // when its partition is the column kernel's; w may then be nullptr, a
@@ -117,13 +117,26 @@ bool gemm_col_supported(int type_id, int64_t row_bytes, int M, int N, int K, con
 hipError_t launch_gemm_col(int type_id, const uint8_t *w, int64_t row_bytes, const uint16_t *x, float *y, int M,
                            int N, int K, hipStream_t stream, const uint8_t *prep = nullptr,
                            int64_t prep_rows = 0);
-// The 128 x 128 tile kernel (gguf_gemm_tile.hip).
+// Whether a shape splits K: when tiles of at most 128 x 128 fill at most half
+// of the CUs.  Only these use the workspace (calls on one handle that do not
+// split may overlap), so the kernels share the rule.
+bool gemm_may_split(int type_id, int M, int N, int K);
+// Q4_K, Q5_K and Q6_K on the fp16 matrix cores (gguf_kq_gemm.hip): K a
+// multiple of 256, x 16-byte and W rows 2-byte aligned.
+bool kq_gemm_supported(int type_id, int64_t row_bytes, int N, int K, const void *w, const void *x);
+size_t kq_gemm_workspace_bytes(int type_id, int M, int N, int K);
+hipError_t launch_kq_gemm(int type_id, const uint8_t *w, int64_t row_bytes, const uint16_t *x, float *y, int M, int N,
+                          int K, hipStream_t stream, float *workspace, size_t workspace_bytes);
+// The 128 x 128 tile kernel of Q8_0 and Q4_0 (gguf_gemm_tile.hip).
 bool gemm_tile_supported(int type_id, int64_t row_bytes, int M, int N, int K, const void *w,
                          const void *x, const void *y);
 size_t gemm_tile_workspace_bytes(int type_id, int M, int N, int K);
 hipError_t launch_gemm_tile(int type_id, const uint8_t *w, int64_t row_bytes, const uint16_t *x,
                             float *y, int M, int N, int K, hipStream_t stream, float *workspace,
                             size_t workspace_bytes);
+// y += the S - 1 partial tiles of mn floats in `part`, in split order (mn a
+// multiple of 4, both 16-byte aligned; S <= 8).
+hipError_t launch_gemm_reduce(const float *part, int S, int64_t mn, float *y, hipStream_t stream);
 
 // Workspace layout of the grouped MoE FFN (byte offsets; gguf_moe.hip).
 struct MoeLayout {

@@ -1,0 +1,270 @@
+// gguf_kq_gemm.hip -- GEMM Y = X . W^T for Q4_K, Q5_K and Q6_K weights on the
+// fp16 matrix cores (gguf_kq_f16.hpp), X bf16 (row-major M x K), fp32
+// accumulate; semantics as gguf_gemm_tile.hip (Q4_K: RT/GgufQ4RawDot.java:331-674).
+//
+// What bounds it: above M ~ 256 the VALU instructions beside the MFMAs.  A
+// wave's 32 columns of a superblock take 18 MFMAs per row tile (16 cycles
+// each) and, at 128 rows, per MFMA 1.6 instructions to widen the codes, 2.1 to
+// scale and convert x and 1.3 to apply d, min and the row scale; timing copies
+// without the x conversion ran Q4_K M = 2048, 14336 x 4096 in 270 us, without
+// the MFMAs in 273 us, whole 345 us.  Below that the latency of a stage (the
+// next superblock's bytes are requested late in it), so small M takes small
+// tiles with the superblocks spread over the waves.
+// Against the bf16 kernel with one FMA per 32 columns and output that this
+// replaces: Q4_K M = 2048 456 -> 345 us (697 TFLOP/s), M = 512 134 -> 97;
+// Q6_K M = 333, 4096 x 14336 183 -> 100 us (its scale groups of 16 took three
+// half-empty MFMAs); Q4_K M = 16 19.5 -> 15.4 us.
+#include "gguf_gemm_plan.hpp"
+#include "gguf_kq_f16.hpp"
+
+namespace gollek {
+
+using namespace kqf;
+
+namespace {
+
+// The x operand of one unit, four rows at a time: lane l takes columns 16 (l &
+// 15) .. + 15 of row 4 j + (l >> 4) (so the loads are whole lines of X), the
+// 16 lanes of a row agree on its scale, and each writes its two fragment
+// pieces and its sub-block's digits.
+template <int T>
+struct XRows {
+    v4u x[2];
+    __device__ __forceinline__ void load(const uint16_t *p) {
+        x[0] = *reinterpret_cast<const v4u *>(p);
+        x[1] = *reinterpret_cast<const v4u *>(p + 8);
+    }
+    // p0, p1: the lane's two pieces, mins: its sub-block's half of a min piece
+    __device__ __forceinline__ void store(uint8_t *p0, uint8_t *p1, uint8_t *mins, float *scale, int lane) const {
+        float v[16], mx = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const uint32_t w = x[i >> 3][(i >> 1) & 3];
+            v[i] = __uint_as_float((i & 1) ? w & 0xFFFF0000u : w << 16);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) mx = fmaxf(fmaxf(mx, fabsf(v[i])), fabsf(v[i + 1]));
+        mx = row_max16(mx);
+        float s, inv, t = 0.0f;
+        kq_row_scale(mx, s, inv);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            uint32_t f[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int e = 8 * h + 4 * (j >> 1) + (j & 1);
+                const f16x2 c = {(_Float16)(v[e] * s), (_Float16)(v[e + 2] * s)};
+                f[j] = as_u(c);
+                if constexpr (KqOperand<T>::kMins) t = __builtin_amdgcn_fdot2(c, splat((_Float16)1.0f), t, false);
+            }
+            *reinterpret_cast<f16x8 *>(h ? p1 : p0) = as_h8(f);
+        }
+        if constexpr (KqOperand<T>::kMins) {
+            t += kq_dpp<0xB1>(t);  // the sub-block's other 16 columns
+            *reinterpret_cast<uint2 *>(mins) = kq_min_digits(t);  // both lanes write the same 8 bytes
+        }
+        if ((lane & 15) == 0) *scale = inv;
+    }
+};
+
+}  // namespace
+
+// A workgroup owns 16 MT rows of X and 32 NW rows of W: NW KW waves as NW
+// column groups of 32 and KW slices of the stage's superblocks.  Each wave
+// converts its rows' share of the next stage's x between its MFMAs.
+template <int T, int MT, int NW, int KW>
+__global__ __launch_bounds__(64 * NW *KW, MT == 1 && NW == 2 ? 4 : 1) void gemm_kq_kernel(const uint8_t *__restrict__ W, int64_t row_bytes,
+                                                              const uint16_t *__restrict__ X, float *__restrict__ Y,
+                                                              int M, int N, int K, int S, float *__restrict__ part) {
+    constexpr int kWaves = NW * KW, UN = MT * KW;
+    constexpr int kTileM = 16 * MT, kTileN = 32 * NW;
+    using U = KqUnit<1>;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[2][UN * U::kBytes];
+
+    const int lane = (int)threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int nw = wave % NW, kw = wave / NW;
+
+    const int tm = (M + kTileM - 1) / kTileM, tn = (N + kTileN - 1) / kTileN;
+    const int G8 = (int)gridDim.x;
+    const int v = (G8 % 8 == 0) ? (int)(blockIdx.x % 8) * (G8 / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
+    const int split = v / (tm * tn);
+    const int t = v - split * tm * tn;
+    const int grp = t / (4 * tn);
+    const int first_m = 4 * grp;
+    const int gm = tm - first_m < 4 ? tm - first_m : 4;
+    const int local = t - grp * 4 * tn;
+    const int m0 = (first_m + local % gm) * kTileM, n0 = (local / gm) * kTileN;
+
+    const int nsb = K / kQK, nst = (nsb + KW - 1) / KW;
+    const int st0 = split * nst / S, st1 = (split + 1) * nst / S;
+
+    const int col0 = n0 + 32 * nw;
+    const uint8_t *wp[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; nt++) {
+        const int r = col0 + 16 * nt + n;
+        wp[nt] = W + (int64_t)(r < N ? r : N - 1) * row_bytes;
+    }
+    f32x4 acc[MT][2];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < 2; nt++) acc[mt][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    auto sb_of = [&](int st) { return st * KW + kw; };
+
+    // This wave's quads of rows: q = wave + kWaves j of the stage's 4 UN.
+    constexpr int kPer = 4 * UN / kWaves;
+    static_assert(4 * UN % kWaves == 0 && kPer <= 4, "whole quads per wave");
+    int xg, xk0, xk1;
+    kq_place<T>(n, xg, xk0, xk1);
+    XRows<T> xr[2];
+    auto load_x = [&](int j, int st) {
+        const int q = wave + kWaves * j, u = q >> 2, sb = st * KW + u / MT;
+        const int r = m0 + 16 * (u % MT) + 4 * (q & 3) + g;
+        // (rows past M repeat row M - 1; their results are not stored)
+        xr[j & 1].load(X + (int64_t)(r < M ? r : M - 1) * K + (int64_t)(sb < nsb ? sb : nsb - 1) * kQK + 16 * n);
+    };
+    auto store_x = [&](int j, int b) {
+        const int q = wave + kWaves * j, u = q >> 2, lr = 4 * (q & 3) + g;
+        uint8_t *const unit = &lds[b][u * U::kBytes];
+        xr[j & 1].store(unit + U::piece(xk0, xg, lr), unit + U::piece(xk1, xg, lr),
+                        unit + U::kMins + 64 * lr + 16 * (n >> 2) + 8 * ((n >> 1) & 1),
+                        reinterpret_cast<float *>(unit + U::kScales) + lr, lane);
+    };
+    load_x(0, st0);
+#pragma unroll
+    for (int j = 0; j < kPer; j++) {
+        if (j + 1 < kPer) load_x(j + 1, st0);
+        store_x(j, 0);
+    }
+    __syncthreads();
+    kq_stages<T, MT, 1>(acc, wp, &lds[0][kw * MT * U::kBytes], UN * U::kBytes, st0, st1, nsb, lane, sb_of,
+                        [&](auto kc, int st, int b) {
+                            constexpr int k = kc.value;
+                            if (k == 0) load_x(0, st);
+                            if (k == 0 && kPer > 1) load_x(1, st);
+                            if (k == 3) store_x(0, b);
+                            if (k == 3 && kPer > 2) load_x(2, st);
+                            if (k == 4 && kPer > 1) store_x(1, b);
+                            if (k == 4 && kPer > 3) load_x(3, st);
+                            if (k == 6 && kPer > 2) store_x(2, b);
+                            if (k == 7 && kPer > 3) store_x(3, b);
+                        });
+
+    if constexpr (KW > 1) {
+        f32x4 *const red = reinterpret_cast<f32x4 *>(lds[0]);
+        if (kw > 0) {
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int nt = 0; nt < 2; nt++) red[((wave * MT + mt) * 2 + nt) * 64 + lane] = acc[mt][nt];
+        }
+        __syncthreads();
+        if (kw > 0) return;
+#pragma unroll
+        for (int k = 1; k < KW; k++)
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int nt = 0; nt < 2; nt++) acc[mt][nt] += red[(((k * NW + nw) * MT + mt) * 2 + nt) * 64 + lane];
+    }
+    float *const out = split == 0 ? Y : part + (int64_t)(split - 1) * M * N;
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int m = m0 + 16 * mt + 4 * g + r;
+#pragma unroll
+            for (int nt = 0; nt < 2; nt++) {
+                const int c = col0 + 16 * nt + n;
+                if (m < M && c < N) out[(int64_t)m * N + c] = acc[mt][nt][r];
+            }
+        }
+}
+
+namespace {
+
+// Fitted per type (gguf_gemm_plan.hpp).
+constexpr GemmPlanCost kQ4KPlans[] = {
+    {1, 1, 4, 2, 3.36f, 2.71f}, {1, 1, 8, 1, 3.73f, 2.95f}, {1, 2, 4, 1, 2.20f, 2.19f},
+    {2, 2, 2, 2, 3.06f, 3.05f}, {2, 2, 4, 1, 3.82f, 3.25f}, {2, 4, 2, 1, 2.55f, 2.47f},
+    {4, 4, 2, 1, 4.02f, 3.73f}, {4, 8, 1, 1, 2.43f, 2.99f}, {6, 8, 1, 1, 3.60f, 3.94f},
+    {8, 8, 1, 1, 4.25f, 4.91f}};
+constexpr GemmSplitCost kQ4KSplit = {1.80f, 0.277f};
+constexpr GemmPlanCost kQ5KPlans[] = {
+    {1, 1, 4, 2, 4.32f, 3.50f}, {1, 1, 8, 1, 4.44f, 3.96f}, {1, 2, 4, 1, 2.97f, 3.03f},
+    {2, 2, 2, 2, 3.96f, 3.81f}, {2, 2, 4, 1, 4.61f, 4.20f}, {2, 4, 2, 1, 3.39f, 3.34f},
+    {4, 4, 2, 1, 4.77f, 4.61f}, {4, 8, 1, 1, 3.64f, 3.79f}, {6, 8, 1, 1, 4.04f, 4.96f},
+    {8, 8, 1, 1, 5.17f, 5.97f}};
+constexpr GemmSplitCost kQ5KSplit = {1.73f, 0.295f};
+constexpr GemmPlanCost kQ6KPlans[] = {
+    {1, 1, 4, 2, 4.59f, 4.39f}, {1, 1, 8, 1, 4.60f, 4.80f}, {1, 2, 4, 1, 3.62f, 4.03f},
+    {2, 2, 2, 2, 4.00f, 4.52f}, {2, 2, 4, 1, 4.51f, 5.15f}, {2, 4, 2, 1, 3.30f, 4.60f},
+    {4, 4, 2, 1, 4.29f, 5.48f}, {4, 8, 1, 1, 3.59f, 5.15f}, {6, 8, 1, 1, 3.89f, 6.27f},
+    {8, 8, 1, 1, 5.83f, 8.54f}};
+constexpr GemmSplitCost kQ6KSplit = {2.43f, 0.297f};
+
+GemmPlan kq_plan(int type_id, int M, int N, int K, size_t ws_bytes) {
+    if (type_id == kQ4_K) return pick_gemm_plan(kQ4KPlans, kQ4KSplit, M, N, K, ws_bytes);
+    if (type_id == kQ5_K) return pick_gemm_plan(kQ5KPlans, kQ5KSplit, M, N, K, ws_bytes);
+    return pick_gemm_plan(kQ6KPlans, kQ6KSplit, M, N, K, ws_bytes);
+}
+
+template <int T, int MT, int NW, int KW>
+void launch(unsigned grid, hipStream_t stream, const uint8_t *w, int64_t row_bytes, const uint16_t *x, float *y,
+            int M, int N, int K, int S, float *part) {
+    hipLaunchKernelGGL((gemm_kq_kernel<T, MT, NW, KW>), dim3(grid), dim3(64 * NW * KW), 0, stream, w, row_bytes, x, y,
+                       M, N, K, S, part);
+}
+
+template <int T, class... A>
+bool launch_plan(const GemmPlan &p, A... a) {
+    const int key = 100 * p.mt + 10 * p.nw + p.kw;
+    switch (key) {
+    case 114: launch<T, 1, 1, 4>(a...); break;
+    case 118: launch<T, 1, 1, 8>(a...); break;
+    case 124: launch<T, 1, 2, 4>(a...); break;
+    case 222: launch<T, 2, 2, 2>(a...); break;
+    case 224: launch<T, 2, 2, 4>(a...); break;
+    case 242: launch<T, 2, 4, 2>(a...); break;
+    case 442: launch<T, 4, 4, 2>(a...); break;
+    case 481: launch<T, 4, 8, 1>(a...); break;
+    case 681: launch<T, 6, 8, 1>(a...); break;
+    case 881: launch<T, 8, 8, 1>(a...); break;
+    default: return false;
+    }
+    return true;
+}
+
+}  // namespace
+
+bool kq_gemm_supported(int type_id, int64_t row_bytes, int N, int K, const void *w, const void *x) {
+    return (type_id == kQ4_K || type_id == kQ5_K || type_id == kQ6_K) && K > 0 && K % kQK == 0 && N > 0 &&
+           ((reinterpret_cast<uintptr_t>(w) | (uintptr_t)row_bytes) & 1u) == 0 &&
+           (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+}
+
+size_t kq_gemm_workspace_bytes(int type_id, int M, int N, int K) {
+    if (!gemm_may_split(type_id, M, N, K)) return 0;
+    return gemm_plan_bytes(kq_plan(type_id, M, N, K, kGemmMaxSplitBytes), M, N);
+}
+
+hipError_t launch_kq_gemm(int type_id, const uint8_t *w, int64_t row_bytes, const uint16_t *x, float *y, int M, int N,
+                          int K, hipStream_t stream, float *workspace, size_t workspace_bytes) {
+    const bool split = workspace != nullptr && gemm_may_split(type_id, M, N, K) && ((int64_t)M * N) % 4 == 0 &&
+                       ((reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(y)) & 15u) == 0;
+    const GemmPlan p = kq_plan(type_id, M, N, K, split ? workspace_bytes : 0);
+    const unsigned grid =
+        (unsigned)(((M + 16 * p.mt - 1) / (16 * p.mt)) * ((N + 32 * p.nw - 1) / (32 * p.nw)) * p.splits);
+    bool ok;
+    if (type_id == kQ4_K) ok = launch_plan<kQ4_K>(p, grid, stream, w, row_bytes, x, y, M, N, K, p.splits, workspace);
+    else if (type_id == kQ5_K) ok = launch_plan<kQ5_K>(p, grid, stream, w, row_bytes, x, y, M, N, K, p.splits, workspace);
+    else ok = launch_plan<kQ6_K>(p, grid, stream, w, row_bytes, x, y, M, N, K, p.splits, workspace);
+    if (!ok) return hipErrorInvalidValue;
+    if (p.splits > 1) return launch_gemm_reduce(workspace, p.splits, (int64_t)M * N, y, stream);
+    return hipGetLastError();
+}
+
+}  // namespace gollek

@@ -99,8 +99,8 @@ def test_gemm_odd_shapes(rows, cols, m):
 
 MATRIX = {syn.Q8_0: syn.q8_0_matrix, syn.Q4_0: syn.q4_0_matrix, syn.Q4_K: syn.q4_k_matrix,
           syn.Q5_K: syn.q5_k_matrix, syn.Q6_K: syn.q6_k_matrix}
-# (Q6_K rows of an odd superblock count, K = 256 here, are not dword
-# multiples and take the fp32 Q6_K kernel instead of the tile kernel.)
+# (Q6_K rows of an odd superblock count, K = 256 here, start on even bytes
+# that are not dwords.)
 TYPES = [syn.Q8_0, syn.Q4_0, syn.Q4_K, syn.Q5_K, syn.Q6_K]
 
 
@@ -265,6 +265,42 @@ def test_gemm_k_quant_unaligned_x_takes_the_generic_kernel(tid):
         assert o.rel_err(y_dev.cpu().numpy(), o.gemm_reference(tid, data, cols, x)) <= GEMM_TOL
     finally:
         dw.close()
+
+
+# The K-quant kernel at the edges of its tiles: row tiles of 16 (M around
+# them, 96 = 6 and 128 = 8 of them), ragged column groups of 32, superblock
+# counts that its waves' slices do not divide, K split over workgroups
+# (N = 64, 1040), weights on even but not dword addresses and y on dword but
+# not 16-byte ones (runs unsplit).  Norm-wise bound: every product is exact, a
+# sum takes 256 additions in the matrix core and K / 256 (at most 17) outside of
+# 2^-24 each, random in sign, with terms up to 8 times the result
+# (d P against dmin PM): 8 * sqrt(273) * 2^-24 = 8e-6.
+@pytest.mark.parametrize("tid", [syn.Q4_K, syn.Q5_K, syn.Q6_K])
+@pytest.mark.parametrize("rows,cols,m", [(33, 256, 5), (64, 4352, 16), (50, 768, 17), (300, 1280, 33), (1040, 2048, 31),
+                                         (2080, 768, 96), (130, 512, 129), (4100, 1024, 333)])
+def test_gemm_k_quant_tiles(tid, rows, cols, m):
+    import torch
+    print(f"[gpu] k-quant gemm type={tid} rows={rows} cols={cols} m={m}", flush=True)
+    data = MATRIX[tid](rows, cols, seed=rows + m)
+    x = syn.activation_bf16(m, cols, seed=rows + m + 1)
+    ref = o.gemm_reference(tid, data, cols, x)
+    raw = np.zeros(data.size + 2, np.uint8)
+    raw[2:] = data.reshape(-1)
+    buf = torch.from_numpy(raw).cuda()
+    xd = torch.from_numpy(x.view(np.int16)).cuda()
+    for w_off, y_off in ((2, 1), (0, 0)):
+        if w_off == 0:
+            buf = torch.from_numpy(np.ascontiguousarray(data.reshape(-1))).cuda()
+        yd = torch.zeros(m * rows + 4, device="cuda")
+        w = ops.DeviceWeight(tid, buf.data_ptr() + w_off, rows, cols)
+        w.gemm_bf16(xd.data_ptr(), m, yd.data_ptr() + 4 * y_off, stream=torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        y = yd.cpu().numpy()
+        got = y[y_off:y_off + m * rows].reshape(m, rows).astype(np.float64)
+        assert np.all(y[:y_off] == 0.0) and np.all(y[y_off + m * rows:] == 0.0)
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        print(f"[gpu] k-quant gemm err={err:.2e}", flush=True)
+        assert err <= 8e-6
 
 
 def test_gemm_rejects_short_buffers():
