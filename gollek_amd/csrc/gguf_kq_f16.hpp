@@ -138,12 +138,19 @@ __device__ __forceinline__ f16x2 splat(_Float16 v) { return f16x2{v, v}; }
 // nibble in place 16 q 2^-24), so widening two of them is one AND and the
 // multiplication by the scale code is also the conversion:
 // q 2^-24 * (sc 2^9) = sc q 2^-15, exact (11 bits above 2^-24).
-template <int T>
+//
+// CENTERED (Q4_K, Q5_K): the operand is sc (q - 8) (Q5_K: q - 16; still exact)
+// and d * 8 (16) * sum_j sc_j * sum(x of sub-block j), one more MFMA like the
+// min term, is added back.  The codes' mean makes up most of an uncentered
+// sum, which then cancels against the min term, so its roundings count about
+// three times as much.
+template <int T, bool CENTERED>
 struct KqOperand {
     static constexpr int kTerms = T == kQ6_K ? 2 : 1;
     static constexpr bool kMins = T != kQ6_K;
+    static constexpr bool kCentered = CENTERED && kMins;
     f16x2 s[T == kQ6_K ? 4 : 2];  // scale codes as operand factors
-    f16x8 bm;
+    f16x8 bm, bs;
     float d, dm;
     __device__ __forceinline__ void head(const KqRaw<T> &r, int g) {
         if constexpr (T == kQ6_K) {
@@ -162,6 +169,10 @@ struct KqOperand {
             s[1] = splat((_Float16)(unsigned short)((scp >> 8) << 5));
             const _Float16 m0 = (_Float16)(unsigned short)(mnp & 0xFFu), m1 = (_Float16)(unsigned short)(mnp >> 8);
             bm = f16x8{m0, m0, m0, (_Float16)0.0f, m1, m1, m1, (_Float16)0.0f};
+            if constexpr (kCentered) {
+                const _Float16 c0 = (_Float16)(unsigned short)(scp & 0xFFu), c1 = (_Float16)(unsigned short)(scp >> 8);
+                bs = f16x8{c0, c0, c0, (_Float16)0.0f, c1, c1, c1, (_Float16)0.0f};
+            }
             d = half_bits_to_float_fast(r.hd.x & 0xFFFFu) * kq_code_scale<T>();
             // no min code set: a non-finite dmin stays out
             // (RT/GgufKQuantLayout.java:67-69)
@@ -200,8 +211,14 @@ struct KqOperand {
                     u0 |= up ? (h << 7) & 0x01000100u : (h << 4) & 0x00100010u;
                     u1 |= up ? (h >> 1) & 0x01000100u : (h >> 4) & 0x00100010u;
                 }
-                lo[2 * t] = as_u(as_h2(u0) * s[up]);
-                lo[2 * t + 1] = as_u(as_h2(u1) * s[up]);
+                if constexpr (kCentered) {  // s = sc 2^9 (low) or sc 2^5: -8 sc 2^-15, Q5_K -16 sc 2^-15
+                    const f16x2 c = s[up] * splat((_Float16)((up ? -0x1p-17f : -0x1p-21f) * (T == kQ5_K ? 2.0f : 1.0f)));
+                    lo[2 * t] = as_u(__builtin_elementwise_fma(as_h2(u0), s[up], c));
+                    lo[2 * t + 1] = as_u(__builtin_elementwise_fma(as_h2(u1), s[up], c));
+                } else {
+                    lo[2 * t] = as_u(as_h2(u0) * s[up]);
+                    lo[2 * t + 1] = as_u(as_h2(u1) * s[up]);
+                }
             }
         }
         b[0] = as_h8(lo);
@@ -275,11 +292,11 @@ __device__ __forceinline__ void static_for(F &&f) {
 // replace this stage's after their last use, in step 6 (requested a stage
 // ahead into registers of their own they cost the small tiles a workgroup per
 // CU: Q4_K M = 16, 14336 x 4096, 15.0 against 17.7 us).
-template <int T, int MT, int DIGITS, class SbOf, class Produce>
+template <int T, int MT, int DIGITS, bool CENTERED, class SbOf, class Produce>
 __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *const (&wp)[2], const uint8_t *units,
                                           int flip, int st0, int st1, int nsb, int lane, SbOf &&sb_of,
                                           Produce &&produce) {
-    using Op = KqOperand<T>;
+    using Op = KqOperand<T, CENTERED>;
     using U = KqUnit<DIGITS>;
     constexpr int NT = Op::kTerms;
     constexpr int MH = MT > 4 ? MT / 2 : MT;  // row tiles whose fragments are held at a time
@@ -354,18 +371,27 @@ __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *co
         for (int mt = 0; mt < MT; mt++) {
             const uint8_t *const unit = cur + mt * U::kBytes;
             const f32x4 inv = *reinterpret_cast<const f32x4 *>(unit + U::kScales + 16 * g);
-            f32x4 pm[2];
+            f32x4 pm[2], ps[2];
             if constexpr (Op::kMins) {
                 const f16x8 am = *reinterpret_cast<const f16x8 *>(unit + U::kMins + 64 * n + 16 * g);
 #pragma unroll
-                for (int nt = 0; nt < 2; nt++) pm[nt] = mfma_f16(am, op[nt].bm, zero);
+                for (int nt = 0; nt < 2; nt++) {
+                    pm[nt] = mfma_f16(am, op[nt].bm, zero);
+                    if constexpr (Op::kCentered) ps[nt] = mfma_f16(am, op[nt].bs, zero);
+                }
             }
 #pragma unroll
             for (int nt = 0; nt < 2; nt++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    float v = op[nt].d * p[mt][nt][r];
-                    if constexpr (Op::kMins) v = fmaf(-op[nt].dm, pm[nt][r], v);
+                    float v = p[mt][nt][r];
+                    if constexpr (Op::kCentered) {  // d P + (d 2^-15 8 PS - dmin PM): the small part last
+                        const float c = op[nt].d * (T == kQ5_K ? 0x1p-11f : 0x1p-12f);
+                        v = fmaf(op[nt].d, v, fmaf(c, ps[nt][r], -op[nt].dm * pm[nt][r]));
+                    } else {
+                        v *= op[nt].d;
+                        if constexpr (Op::kMins) v = fmaf(-op[nt].dm, pm[nt][r], v);
+                    }
                     const float c = acc[mt][nt][r];
                     acc[mt][nt][r] = act ? fmaf(inv[r], v, c) : c;
                 }

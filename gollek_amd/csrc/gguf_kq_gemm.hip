@@ -55,11 +55,11 @@ struct XRows {
                 const int e = 8 * h + 4 * (j >> 1) + (j & 1);
                 const f16x2 c = {(_Float16)(v[e] * s), (_Float16)(v[e + 2] * s)};
                 f[j] = as_u(c);
-                if constexpr (KqOperand<T>::kMins) t = __builtin_amdgcn_fdot2(c, splat((_Float16)1.0f), t, false);
+                if constexpr (KqOperand<T, false>::kMins) t = __builtin_amdgcn_fdot2(c, splat((_Float16)1.0f), t, false);
             }
             *reinterpret_cast<f16x8 *>(h ? p1 : p0) = as_h8(f);
         }
-        if constexpr (KqOperand<T>::kMins) {
+        if constexpr (KqOperand<T, false>::kMins) {
             t += kq_dpp<0xB1>(t);  // the sub-block's other 16 columns
             *reinterpret_cast<uint2 *>(mins) = kq_min_digits(t);  // both lanes write the same 8 bytes
         }
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(64 * NW *KW, MT == 1 && NW == 2 ? 4 : 1) void gemm_
         store_x(j, 0);
     }
     __syncthreads();
-    kq_stages<T, MT, 1>(acc, wp, &lds[0][kw * MT * U::kBytes], UN * U::kBytes, st0, st1, nsb, lane, sb_of,
+    kq_stages<T, MT, 1, false>(acc, wp, &lds[0][kw * MT * U::kBytes], UN * U::kBytes, st0, st1, nsb, lane, sb_of,
                         [&](auto kc, int st, int b) {
                             constexpr int k = kc.value;
                             if (k == 0) load_x(0, st);

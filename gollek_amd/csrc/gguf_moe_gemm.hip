@@ -81,7 +81,7 @@ __global__ __launch_bounds__(256) void moe_records_kernel(const float *v, int ro
         for (int d = 0; d < 2; d++)
             *reinterpret_cast<f16x8 *>(dst + 512 * (kk[h] >> 2) + 256 * d + 16 * (4 * (kk[h] & 3) + g)) = as_h8(f[d]);
     }
-    if constexpr (KqOperand<T>::kMins) {
+    if constexpr (KqOperand<T, true>::kMins) {
         t += kq_dpp<0xB1>(t);  // the sub-block's other 16 columns
         *reinterpret_cast<uint2 *>(mins + rs * kTailBytes + 16 * (n >> 2) + 8 * ((n >> 1) & 1)) = kq_min_digits(t);
     }
@@ -128,13 +128,13 @@ __device__ __forceinline__ void moe_item(const uint8_t *const (&wp)[2], int nsb,
         }
     };
     auto load_tail = [&](int sb) {
-        if constexpr (KqOperand<T>::kMins)
+        if constexpr (KqOperand<T, true>::kMins)
             if (tid < 64 * MT)
                 tail = *reinterpret_cast<const v4u *>(mins + ((int64_t)rows[tid >> 2] * nsb + sb) * kTailBytes + 16 * (tid & 3));
         if (tid < 16 * MT) sc = scales[(int64_t)rows[tid] * nsb + sb];
     };
     auto store_tail = [&](int b) {
-        if constexpr (KqOperand<T>::kMins)
+        if constexpr (KqOperand<T, true>::kMins)
             if (tid < 64 * MT)
                 *reinterpret_cast<v4u *>(lds + (b * MT + (tid >> 6)) * U::kBytes + U::kMins + 16 * (tid & 63)) = tail;
         if (tid < 16 * MT)
@@ -148,7 +148,7 @@ __device__ __forceinline__ void moe_item(const uint8_t *const (&wp)[2], int nsb,
     }
     store_tail(0);
     __syncthreads();
-    kq_stages<T, MT, 2>(acc, wp, lds, MT * U::kBytes, 0, nsb, nsb, lane, [](int st) { return st; },
+    kq_stages<T, MT, 2, true>(acc, wp, lds, MT * U::kBytes, 0, nsb, nsb, lane, [](int st) { return st; },
                         [&](auto kc, int sb, int b) {
                             constexpr int k = kc.value, per = 8 / kBatches;
                             if constexpr (k == 0) load_tail(sb);
