@@ -14,19 +14,12 @@
 // fp32 result before accumulation -- the reference's own block structure.
 // Rounding q * d to bf16 instead would cost ~1e-3 relative error per weight.
 //
-// Kernels.  Q8_0 with M <= 32: gemm_q8_0_bf16_skinny_kernel (16-row column
-// tiles, K split over the waves, one buffer->LDS ring per wave).  Q8_0, Q4_0
-// and Q4_K with K a multiple of 256 otherwise: the 128 x 128 tile kernel of
-// gguf_gemm_tile.hip.  Other shapes: gemm_q8_0_bf16_kernel, where a
-// workgroup of 4 waves owns a BM x BN tile of Y; the waves split it WM x WN
-// and, when WK > 1, also split each K stage (the partial tiles are summed
-// through LDS at the end).  Each stage moves KB = 64 * WK columns of X (bf16)
-// and W (Q8_0 block pairs, 68 aligned bytes, realigned and widened to bf16
-// once per workgroup) into double-buffered LDS; one barrier per stage.  Any
-// remaining shape or alignment: one thread per output (gemm_q8_0_generic_kernel,
-// gemm_generic_kernel).
-#include <type_traits>
-
+// Kernels.  Q8_0 with M <= 32 and K a multiple of 256:
+// gemm_q8_0_bf16_skinny_kernel (16-row column tiles, K split over the waves,
+// one buffer->LDS ring per wave).  Other Q8_0 and Q4_0: gguf_gemm_tile.hip.
+// K-quants: gguf_kq_gemm.hip.  Buffers aligned for neither: Q6_K in fp32
+// tiles, anything else one thread per output (gemm_q8_0_generic_kernel,
+// gemm_generic_kernel, gemm_kquant_generic_kernel).
 #include "gguf_block_dot.hpp"
 #include "gguf_blocks.hpp"
 #include "gguf_dot4.hpp"
@@ -39,8 +32,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kPad = 8;  // bf16 elements of row padding in LDS (bank spread)
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -55,197 +46,6 @@ __device__ __forceinline__ void i8x4_to_bf16(uint32_t w, uint32_t &a, uint32_t &
     a = pack_bf16x2((float)(int)(int8_t)(w & 0xFFu), (float)(int)(int8_t)((w >> 8) & 0xFFu));
     b = pack_bf16x2((float)(int)(int8_t)((w >> 16) & 0xFFu), (float)(int)(int8_t)(w >> 24));
 }
-
-template <int BM, int BN, int KB>
-struct Stage {
-    uint16_t x[BM][KB + kPad];
-    uint16_t w[BN][KB + kPad];
-    float d[BN][KB / 32];
-};
-
-// Registers holding one stage's global data before it is written to LDS.
-template <int XCH, int WIT>
-struct StageRegs {
-    uint4 x[XCH];
-    uint32_t q[WIT][5];
-    uint32_t dw[WIT];
-};
-
-}  // namespace
-
-template <int BM, int BN, int WM, int WN, int WK>
-__global__ __launch_bounds__(256) void gemm_q8_0_bf16_kernel(const uint8_t *__restrict__ W,
-                                                             int64_t row_bytes,
-                                                             const uint16_t *__restrict__ X,
-                                                             float *__restrict__ Y, int M, int N,
-                                                             int K) {
-    constexpr int KB = 64 * WK;              // K columns per stage
-    constexpr int NBLK = KB / 32;            // Q8_0 blocks per row per stage
-    constexpr int MT = WM / 16, NT = WN / 16;
-    constexpr int WAVES_M = BM / WM, WAVES_N = BN / WN;
-    static_assert(WAVES_M * WAVES_N * WK == 4, "four waves per workgroup");
-    constexpr int XCHUNKS = BM * KB / 8;     // 16-byte chunks of X per stage
-    constexpr int XCH = (XCHUNKS + 255) / 256;
-    constexpr int WITEMS = BN * NBLK * 2;    // (row, block, half) items per stage
-    constexpr int WIT = (WITEMS + 255) / 256;
-    using StageT = Stage<BM, BN, KB>;
-    __shared__ StageT st[2];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int wk = wave % WK;
-    const int wn = (wave / WK) % WAVES_N;
-    const int wm = wave / (WK * WAVES_N);
-    const int m0 = blockIdx.y * BM;
-    const int n0 = blockIdx.x * BN;
-    const int nstages = K / KB;
-
-    StageRegs<XCH, WIT> R;
-
-    auto load_global = [&](int s) {
-        const int k0 = s * KB;
-#pragma unroll
-        for (int i = 0; i < XCH; i++) {
-            const int c = tid + 256 * i;
-            const int r = c / (KB / 8), kc = c % (KB / 8);
-            R.x[i] = make_uint4(0u, 0u, 0u, 0u);
-            if (c < XCHUNKS && m0 + r < M)
-                R.x[i] = *reinterpret_cast<const uint4 *>(X + (int64_t)(m0 + r) * K + k0 + 8 * kc);
-        }
-#pragma unroll
-        for (int i = 0; i < WIT; i++) {
-            const int it = tid + 256 * i;
-            // item -> (row n, block bi, half u): half u holds quants 16u..16u+15
-            const int n = it / (NBLK * 2);
-            const int rem = it % (NBLK * 2);
-            const int bi = rem >> 1, u = rem & 1;
-            // Byte offset of block bi inside the row's stage segment; blocks
-            // come in 68-byte pairs, so pair starts are 4-byte aligned.
-            const int pair = bi >> 1, odd = bi & 1;
-            const uint32_t *base = reinterpret_cast<const uint32_t *>(
-                W + (int64_t)(n0 + n) * row_bytes + (int64_t)(k0 / 64) * 68 + 68 * pair);
-            // Quant bytes of block (pair, odd), half u: odd ? 36 + 16u : 2 + 16u.
-            const int first = odd ? 9 + 4 * u : 4 * u;  // first dword covering them
-            if (it < WITEMS) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) R.q[i][j] = base[first + j];
-                // even blocks start 2 bytes into a dword and need a fifth one
-                R.q[i][4] = odd ? 0u : base[first + 4];
-                R.dw[i] = base[odd ? 8 : 0];
-            }
-        }
-    };
-
-    auto store_lds = [&](int buf) {
-        StageT &S = st[buf];
-#pragma unroll
-        for (int i = 0; i < XCH; i++) {
-            const int c = tid + 256 * i;
-            const int r = c / (KB / 8), kc = c % (KB / 8);
-            if (c < XCHUNKS) *reinterpret_cast<uint4 *>(&S.x[r][8 * kc]) = R.x[i];
-        }
-#pragma unroll
-        for (int i = 0; i < WIT; i++) {
-            const int it = tid + 256 * i;
-            if (it >= WITEMS) continue;
-            const int n = it / (NBLK * 2);
-            const int rem = it % (NBLK * 2);
-            const int bi = rem >> 1, u = rem & 1;
-            const int odd = bi & 1;
-            uint32_t qd[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                qd[j] = odd ? R.q[i][j] : __builtin_amdgcn_alignbyte(R.q[i][j + 1], R.q[i][j], 2);
-            uint32_t o[8];
-#pragma unroll
-            for (int j = 0; j < 4; j++) i8x4_to_bf16(qd[j], o[2 * j], o[2 * j + 1]);
-            uint4 *dst = reinterpret_cast<uint4 *>(&S.w[n][32 * bi + 16 * u]);
-            dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
-            dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
-            if (u == 0) S.d[n][bi] = half_bits_to_float_fast(odd ? (R.dw[i] >> 16) : R.dw[i]);
-        }
-    };
-
-    f32x4 acc[MT][NT];
-#pragma unroll
-    for (int a = 0; a < MT; a++)
-#pragma unroll
-        for (int b = 0; b < NT; b++) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    load_global(0);
-    store_lds(0);
-    __syncthreads();
-    const int lr = lane & 15;       // operand row (A) / column (B) within a 16-tile
-    const int lk = 8 * (lane >> 4); // operand k offset within a 32-block
-    for (int s = 0; s < nstages; s++) {
-        const int buf = s & 1;
-        if (s + 1 < nstages) load_global(s + 1);
-        const StageT &S = st[buf];
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            const int kb = 2 * wk + b;  // block index inside the stage
-            bf16x8 A[MT], B[NT];
-            float dsc[NT];
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++)
-                A[mt] = *reinterpret_cast<const bf16x8 *>(&S.x[wm * WM + 16 * mt + lr][32 * kb + lk]);
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                B[nt] = *reinterpret_cast<const bf16x8 *>(&S.w[wn * WN + 16 * nt + lr][32 * kb + lk]);
-                dsc[nt] = S.d[wn * WN + 16 * nt + lr][kb];
-            }
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++) {
-                    const f32x4 t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        A[mt], B[nt], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                    for (int v = 0; v < 4; v++) acc[mt][nt][v] = fmaf(dsc[nt], t[v], acc[mt][nt][v]);
-                }
-        }
-        if (s + 1 < nstages) store_lds(buf ^ 1);
-        __syncthreads();
-    }
-
-    // D layout of a 16x16 tile: lane holds column lane & 15, rows 4 (lane >> 4) + v.
-    if (WK > 1) {
-        float *red = reinterpret_cast<float *>(&st[0]);  // stages are free after the loop
-        if (wk != 0) {
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        red[(((wave * MT + mt) * NT + nt) * 4 + v) * 64 + lane] = acc[mt][nt][v];
-        }
-        __syncthreads();
-        if (wk != 0) return;
-#pragma unroll
-        for (int o = 1; o < WK; o++)
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        acc[mt][nt][v] += red[((((wave + o) * MT + mt) * NT + nt) * 4 + v) * 64 + lane];
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int m = m0 + wm * WM + 16 * mt + 4 * (lane >> 4) + v;
-                const int n = n0 + wn * WN + 16 * nt + lr;
-                if (m < M) Y[(int64_t)m * N + n] = acc[mt][nt][v];
-            }
-}
-
-namespace {
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
@@ -696,19 +496,6 @@ __global__ __launch_bounds__(256) void gemm_q6k_f32_kernel(const uint8_t *__rest
     }
 }
 
-namespace {
-
-template <int BM, int BN, int WM, int WN, int WK>
-hipError_t launch_tiled(const uint8_t *w, int64_t row_bytes, const uint16_t *x, float *y, int M,
-                        int N, int K, hipStream_t stream) {
-    const dim3 grid(N / BN, (M + BM - 1) / BM);
-    hipLaunchKernelGGL((gemm_q8_0_bf16_kernel<BM, BN, WM, WN, WK>), grid, dim3(256), 0, stream, w,
-                       row_bytes, x, y, M, N, K);
-    return hipGetLastError();
-}
-
-}  // namespace
-
 size_t gemm_workspace_bytes(int type_id, int M, int N, int K) {
     if (type_id == kQ8_0 && M <= 32) return 0;  // the skinny kernel
     if (type_id == kQ4_K || type_id == kQ5_K || type_id == kQ6_K) return kq_gemm_workspace_bytes(type_id, M, N, K);
@@ -760,18 +547,10 @@ hipError_t launch_gemm_bf16(int type_id, const uint8_t *w, int64_t row_bytes, co
     // K-quants: codes widened in registers, fp16 matrix cores.
     if (kq_gemm_supported(type_id, row_bytes, N, K, w, x))
         return launch_kq_gemm(type_id, w, row_bytes, x, y, M, N, K, stream, workspace, workspace_bytes);
-    // 128 x 128 tiles for Q8_0 and Q4_0 (K a multiple of 256).
-    if (gemm_tile_supported(type_id, row_bytes, M, N, K, w, x, y))
+    // Q8_0 and Q4_0: tiles of 16 .. 128 x 128.
+    if (gemm_tile_supported(type_id, row_bytes, M, N, K, w, x))
         return launch_gemm_tile(type_id, w, row_bytes, x, y, M, N, K, stream, workspace, workspace_bytes);
     // Other shapes and alignments.
-    if (type_id == kQ8_0 && aligned) {
-        if (M <= 16 && N % 16 == 0 && K % 256 == 0)
-            return launch_tiled<16, 16, 16, 16, 4>(w, row_bytes, x, y, M, N, K, stream);
-        if (M <= 128 && N % 16 == 0 && K % 64 == 0)
-            return launch_tiled<128, 16, 32, 16, 1>(w, row_bytes, x, y, M, N, K, stream);
-        if (N % 64 == 0 && K % 64 == 0)
-            return launch_tiled<128, 64, 64, 32, 1>(w, row_bytes, x, y, M, N, K, stream);
-    }
     // Q6_K with 4-byte aligned X rows: the fp32 matrix-core kernel, tiles of
     // 16 W rows and 16 / 32 / 64 X rows, or 64 x 64 tiles when those still
     // give every CU two workgroups (fewer re-reads of X).

@@ -229,7 +229,9 @@ __device__ __forceinline__ void ops_wait_row(int i, Ops &o) {
 }  // namespace
 
 // One 16 MT x 128 tile of Y (or of split `split`'s partial sum) per workgroup.
-template <int T, int MT>
+// RAGGED: K is any multiple of 32 and rows may start 2 bytes past a dword (kept
+// apart: the address masks and the skipped half stage cost whole-round K 1 to 2 %).
+template <int T, int MT, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__restrict__ W,
                                                             int64_t row_bytes,
                                                             const uint16_t *__restrict__ X,
@@ -260,11 +262,16 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
     const int gm = tm - first_m < 4 ? tm - first_m : 4;
     const int local = t - grp * 4 * tn;
     const int m0 = (first_m + local % gm) * kTileM, n0 = (local / gm) * kTileN;
-    const int nst = K / 64 / S;  // stages of this split (a multiple of 4)
+    // Stages of this split (S > 1: a multiple of 4).  With an odd number of
+    // blocks the last stage holds one, and the waves of the second block skip
+    // it (its X and W bytes are the next row's, or zeros).
+    const int nst = (K + 63) / 64 / S;
     const int s0 = split * nst;
+    const bool half_last = RAGGED && (K & 32) != 0;
 
     // Buffers from the split's first column; rows past M / N and bytes past
-    // the end read as zeros.
+    // the end read as zeros (W's end rounded up to a dword: a buffer load drops
+    // the dword that its end cuts).
     const int mrows = M - m0 < kTileM ? M - m0 : kTileM;
     const int nrows = N - n0 < kTileN ? N - n0 : kTileN;
     const int64_t w_split = (int64_t)s0 * R::kStageBytes;
@@ -272,7 +279,7 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
         reinterpret_cast<const uint8_t *>(X) + (int64_t)m0 * K * 2 + (int64_t)s0 * 128,
         (uint32_t)((int64_t)mrows * K * 2 - (int64_t)s0 * 128));
     const __amdgpu_buffer_rsrc_t wr = wave_buffer(W + (int64_t)n0 * row_bytes + w_split,
-                                                  (uint32_t)((int64_t)nrows * row_bytes - w_split));
+                                                  (uint32_t)(((int64_t)nrows * row_bytes - w_split + 3) & ~(int64_t)3));
 
     // ---- loads of a stage (loader waves 8 and 9) ---------------------------
     // X: loader l moves LDS chunks p = 64 (MT l + i) + lane (i < MT): row p / 8
@@ -296,8 +303,9 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
             const int j = ldr + 2 * i;
             const int q = 64 * j + lane;
             const int row = q / R::kChunks, part = q - row * R::kChunks;
-            const uint32_t off =
-                (uint32_t)row * (uint32_t)row_bytes + (uint32_t)(16 * part) + (uint32_t)(R::kStageBytes * ls);
+            // from the dword at or before the row's bytes
+            const uint32_t off = (((uint32_t)row * (uint32_t)row_bytes) & (RAGGED ? ~2u : ~0u)) +
+                                 (uint32_t)(16 * part) + (uint32_t)(R::kStageBytes * ls);
             dma16(wr, rs + 1024 * j, off);
         }
     };
@@ -314,20 +322,15 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
     const uint32_t wrow = ring_base + (uint32_t)(kXBytes + G::kPitch * (32 * nq + lr));
     // Per-lane code and scale offsets in a row's raw bytes, and the byte shift
     // that realigns the codes.
-    uint32_t qoff, soff, qsh, nsh;
-    if constexpr (T == kQ8_0) {
-        // block kg's 8 codes of lane group lk at byte 2 + 34 kg + 8 lk; scale in dword 8 kg
-        qoff = (uint32_t)(4 * (kg ? 9 + 2 * lk : 2 * lk));
-        qsh = kg ? 0u : 2u;
-        soff = (uint32_t)(32 * kg);
-        nsh = 16u * (uint32_t)kg;  // scale half
-    } else {
-        // 8 bytes of block kg at byte 2 + 18 kg + 8 (lk & 1); nibble lk >> 1; scale in dword 4 kg
-        qoff = (uint32_t)(4 * (kg ? 5 + 2 * (lk & 1) : 2 * (lk & 1)));
-        qsh = kg ? 0u : 2u;
-        soff = (uint32_t)(16 * kg);
-        nsh = 16u * (uint32_t)kg;
-    }
+    // Block kg at byte 34 kg (Q4_0: 18 kg) of the row's stage bytes, which stand
+    // 2 bytes past a dword in the odd rows of an odd block count (rows 16
+    // apart alike: the same for both column tiles).  Codes from byte 2: Q8_0's 8
+    // of lane group lk from 8 lk, Q4_0's 8 bytes from 8 (lk & 1).
+    const uint32_t at = (uint32_t)((T == kQ8_0 ? kQ8BlockBytes : kQ4BlockBytes) * kg) +
+                        (RAGGED ? ((uint32_t)lr * (uint32_t)row_bytes) & 2u : 0u);
+    const uint32_t qat = at + 2u + (uint32_t)(8 * (T == kQ8_0 ? lk : lk & 1));
+    const uint32_t qoff = qat & ~3u, qsh = qat & 3u;
+    const uint32_t soff = at & ~3u, nsh = 8u * (at & 3u);  // the scale's dword and half
     const int nib = 4 * (lk >> 1);  // nibble shift (Q4_0)
 
     f32x4 acc[MT][2];
@@ -413,7 +416,7 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
     } else {
         for (int s = 0; s < nst; s++) {
             compute_barrier();
-            compute(s);
+            if (!(half_last && kg == 1 && s == nst - 1)) compute(s);  // uniform
         }
     }
 
@@ -463,7 +466,7 @@ __global__ __launch_bounds__(kThreads) void gemm_tile_kernel(const uint8_t *__re
         if (m >= M || n >= N) continue;
         const float4 val = *reinterpret_cast<const float4 *>(stage + row * kStagePitch + col);
         float *const dst = out + (int64_t)m * N + n;
-        if ((N & 3) == 0) {
+        if ((N & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
             // nontemporal: the tile is not read again by this kernel
             __builtin_nontemporal_store(f32x4{val.x, val.y, val.z, val.w}, reinterpret_cast<f32x4 *>(dst));
         } else {
@@ -498,13 +501,33 @@ __global__ __launch_bounds__(256) void gemm_tile_reduce_kernel(const float *__re
 
 namespace {
 
-// Row tiles of X per workgroup: the smallest of 1, 2, 4, 8 that covers M, so
-// that small M computes no padding rows.  Q8_0 up to M = 128 with so few
-// column tiles that 128-row tiles would split K eight ways takes 64-row
-// tiles split four ways instead: three partial tiles per output in place of
-// seven (M = 128, N = 4096: 18.7 against 19.7 us; the Q4_0 tiles at N =
-// 14336 measured slower with 64 rows).
-int tile_mt(int type_id, int M, int N) {
+// Row tiles of X per workgroup.  Shapes that may split K (whole 256-column
+// rounds): the smallest of 1, 2, 4, 8 that covers M, so that small M computes
+// no padding rows.  Q8_0 up to M = 128 with so few column tiles that 128-row
+// tiles would split K eight ways takes 64-row tiles split four ways instead:
+// three partial tiles per output in place of seven (M = 128, N = 4096: 18.7
+// against 19.7 us; the Q4_0 tiles at N = 14336 measured slower with 64 rows).
+// Other K run unsplit (they always have: see gemm_may_split): the tile height with the shortest rounds over the CUs
+// (a stage of 1, 2, 4 or 8 row tiles takes about 0.46, 0.54, 0.69 and 0.95 us,
+// a tile's start and end 3 us).  N = 5760, K = 2880, M = 100: 20.6 us, 40.9 on the
+// converted-copy kernel these shapes took before; K = 2912, M = 256, N = 4000:
+// 23 us, 1220 with one thread per output.
+int tile_mt(int type_id, int M, int N, int K) {
+    if (K % 256 != 0) {
+        constexpr float kStage[4] = {0.46f, 0.54f, 0.69f, 0.95f};
+        int best = 8;
+        float best_us = 0.0f;
+        for (int i = 0; i < 4; i++) {
+            const int mt = 1 << i;
+            const int64_t tiles = (int64_t)((M + 16 * mt - 1) / (16 * mt)) * ((N + kTileN - 1) / kTileN);
+            const float us = (float)((tiles + device_cus() - 1) / device_cus()) * (3.0f + kStage[i] * ((K + 63) / 64));
+            if (i == 0 || us < best_us) {
+                best = mt;
+                best_us = us;
+            }
+        }
+        return best;
+    }
     if (M <= 16) return 1;
     if (M <= 32) return 2;
     if (M <= 64) return 4;
@@ -513,12 +536,12 @@ int tile_mt(int type_id, int M, int N) {
 }
 
 int tile_splits(int type_id, int M, int N, int K, size_t workspace_bytes) {
-    const int tm = 16 * tile_mt(type_id, M, N);
+    const int tm = 16 * tile_mt(type_id, M, N, K);
     const int tiles = (M + tm - 1) / tm * ((N + kTileN - 1) / kTileN);
     const int nst = K / 64;
     // A split holds a whole number of four-stage rounds.
     int S = 1;
-    while (S < 8 && tiles * 2 * S <= device_cus() && nst % (8 * S) == 0 &&
+    while (S < 8 && K % 256 == 0 && tiles * 2 * S <= device_cus() && nst % (8 * S) == 0 &&
            (size_t)(2 * S - 1) * M * N * sizeof(float) <= workspace_bytes)
         S *= 2;
     return S;
@@ -526,12 +549,11 @@ int tile_splits(int type_id, int M, int N, int K, size_t workspace_bytes) {
 
 }  // namespace
 
-bool gemm_tile_supported(int type_id, int64_t row_bytes, int M, int N, int K, const void *w,
-                         const void *x, const void *y) {
+bool gemm_tile_supported(int type_id, int64_t row_bytes, int M, int N, int K, const void *w, const void *x) {
     if (type_id != kQ8_0 && type_id != kQ4_0) return false;
-    if (M <= 0 || N <= 0 || K % 256 != 0) return false;
-    if (((reinterpret_cast<uintptr_t>(w) | (uintptr_t)row_bytes) & 3u) != 0) return false;
-    if ((reinterpret_cast<uintptr_t>(x) & 15u) != 0 || (reinterpret_cast<uintptr_t>(y) & 15u) != 0) return false;
+    if (M <= 0 || N <= 0 || K <= 0 || K % 32 != 0) return false;
+    if ((reinterpret_cast<uintptr_t>(w) & 3u) != 0 || ((uintptr_t)row_bytes & 1u) != 0) return false;
+    if ((reinterpret_cast<uintptr_t>(x) & 15u) != 0) return false;
     // 32-bit buffer offsets: a tile's rows of X and W
     return (int64_t)kTileMMax * K * 2 < ((int64_t)1 << 31) && (int64_t)kTileN * row_bytes < ((int64_t)1 << 31);
 }
@@ -548,25 +570,23 @@ hipError_t launch_gemm_tile(int type_id, const uint8_t *w, int64_t row_bytes, co
                             size_t workspace_bytes) {
     if (M <= 0) return hipSuccess;
     int S = tile_splits(type_id, M, N, K, workspace != nullptr ? workspace_bytes : 0);
-    if (((int64_t)M * N) % 4 != 0 || (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) S = 1;
-    const int mt = tile_mt(type_id, M, N), tm = 16 * mt;
+    if (((int64_t)M * N) % 4 != 0 ||
+        ((reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(y)) & 15u) != 0)
+        S = 1;
+    const int mt = tile_mt(type_id, M, N, K), tm = 16 * mt;
     const unsigned tiles = (unsigned)(((M + tm - 1) / tm) * ((N + kTileN - 1) / kTileN));
     const dim3 grid(tiles * (unsigned)S), block(kThreads);
     float *part = S > 1 ? workspace : nullptr;
-#define GOLLEK_TILE_LAUNCH(TY)                                                                        \
-    do {                                                                                              \
-        if (mt == 1)                                                                                  \
-            hipLaunchKernelGGL((gemm_tile_kernel<TY, 1>), grid, block, 0, stream, w, row_bytes, x, y, M, N, \
-                               K, S, part);                                                           \
-        else if (mt == 2)                                                                             \
-            hipLaunchKernelGGL((gemm_tile_kernel<TY, 2>), grid, block, 0, stream, w, row_bytes, x, y, M, N, \
-                               K, S, part);                                                           \
-        else if (mt == 4)                                                                             \
-            hipLaunchKernelGGL((gemm_tile_kernel<TY, 4>), grid, block, 0, stream, w, row_bytes, x, y, M, N, \
-                               K, S, part);                                                           \
-        else                                                                                          \
-            hipLaunchKernelGGL((gemm_tile_kernel<TY, 8>), grid, block, 0, stream, w, row_bytes, x, y, M, N, \
-                               K, S, part);                                                           \
+    const bool ragged = K % 64 != 0 || (row_bytes & 3) != 0;
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, w, row_bytes, x, y, M, N, K, S, part);
+    };
+#define GOLLEK_TILE_LAUNCH(TY)                                                                              \
+    do {                                                                                                    \
+        if (mt == 1) ragged ? run(&gemm_tile_kernel<TY, 1, true>) : run(&gemm_tile_kernel<TY, 1, false>);   \
+        else if (mt == 2) ragged ? run(&gemm_tile_kernel<TY, 2, true>) : run(&gemm_tile_kernel<TY, 2, false>); \
+        else if (mt == 4) ragged ? run(&gemm_tile_kernel<TY, 4, true>) : run(&gemm_tile_kernel<TY, 4, false>); \
+        else ragged ? run(&gemm_tile_kernel<TY, 8, true>) : run(&gemm_tile_kernel<TY, 8, false>);           \
     } while (0)
     switch (type_id) {
     case kQ8_0:

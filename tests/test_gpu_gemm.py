@@ -303,6 +303,36 @@ def test_gemm_k_quant_tiles(tid, rows, cols, m):
         assert err <= 8e-6
 
 
+# Q8_0 / Q4_0 on the tile kernel with K a multiple of 32 only: an odd number of
+# blocks (the last 64-column stage holds one; odd rows start on even bytes that
+# are no dword), one block, every tile height, ragged N, y on a dword address.
+# Norm-wise bound: exact products, K / 32 (at most 91) roundings of 2^-24, random
+# in sign, of terms no larger than the result's norm: 10 * 2^-24 and twice
+# that for the matrix core's own sums.
+@pytest.mark.parametrize("tid", [syn.Q8_0, syn.Q4_0])
+@pytest.mark.parametrize("rows,cols,m", [(33, 32, 1), (130, 96, 17), (300, 2912, 5), (129, 1056, 64), (1000, 864, 65),
+                                         (4000, 2912, 130), (5760, 2880, 100), (70, 64, 600)])
+def test_gemm_ragged_k(tid, rows, cols, m):
+    import torch
+    print(f"[gpu] ragged gemm type={tid} rows={rows} cols={cols} m={m}", flush=True)
+    data = MATRIX[tid](rows, cols, seed=rows + m)
+    x = syn.activation_bf16(m, cols, seed=rows + m + 1)
+    ref = o.gemm_reference(tid, data, cols, x)
+    buf = torch.from_numpy(np.ascontiguousarray(data.reshape(-1))).cuda()
+    xd = torch.from_numpy(x.view(np.int16)).cuda()
+    for y_off in (0, 1):
+        yd = torch.zeros(m * rows + 4, device="cuda")
+        w = ops.DeviceWeight(tid, buf.data_ptr(), rows, cols)
+        w.gemm_bf16(xd.data_ptr(), m, yd.data_ptr() + 4 * y_off, stream=torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        y = yd.cpu().numpy()
+        got = y[y_off:y_off + m * rows].reshape(m, rows).astype(np.float64)
+        assert np.all(y[:y_off] == 0.0) and np.all(y[y_off + m * rows:] == 0.0)
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        print(f"[gpu] ragged gemm err={err:.2e}", flush=True)
+        assert err <= 20 * 2.0 ** -24
+
+
 def test_gemm_rejects_short_buffers():
     data = syn.q8_0_matrix(16, 64, seed=1)
     t = ops.GgufTensor("w", (64, 16), syn.Q8_0, data.reshape(-1))
