@@ -200,11 +200,9 @@ hipError_t launch_moe_gemm(int gate_type, int down_type, const uint8_t *gate, co
                            int top_k, float *out, uint8_t *ws, hipStream_t stream);
 
 // Pieces of the MoE pipeline shared by its implementations (gguf_moe.hip,
-// gguf_moe_mfma.hip, gguf_moe_gemm.hip): routing (meta layout of moe_layout;
-// group > 0: also the grouped GEMM's items of at most `group` routes) and
-// the route-order combine.
-hipError_t launch_moe_route(const int32_t *ids, const float *wts, int P, int E, int group, int32_t *meta,
-                            int2 *items, hipStream_t stream);
+// gguf_moe_mfma.hip, gguf_moe_gemm.hip): routing (meta layout of moe_layout)
+// and the route-order combine.
+hipError_t launch_moe_route(const int32_t *ids, const float *wts, int P, int E, int32_t *meta, hipStream_t stream);
 hipError_t launch_moe_combine(const int32_t *ids, const float *wts, const float *ypair, int T,
                               int top_k, int H, int E, float *out, hipStream_t stream);
 // MoE router (gguf_moe_router.hip): logits [T, E] -> ids / wts [T, K] with

@@ -18,15 +18,16 @@
 // tile), so its loads' latency shows; small tiles keep several workgroups on
 // a CU.  128 experts x 768, hidden 2048, Q4_K gate / up, Q6_K down, 256 tokens x
 // top-8: 717 us on the passes of gguf_moe_mfma.hip, 204 here (gate/up 96 us for
-// 226 MB, down 100 us for 165 MB, the other five launches 29 us); 32 x 1280,
+// 226 MB, down 100 us for 165 MB, the other launches 24 us); 32 x 1280,
 // hidden 2816, 256 tokens x top-4: 2435 us on the row kernels, 157 here.
 //
 // Launches: routing (a list of (expert, first route) items of at most 16 MT
-// routes), x records, gate/up (h), h records, down (a row per route), combine
+// routes) with x's records, gate/up (h), h records, down (a row per route), combine
 // in route order.
 #include "gguf_dot4.hpp"
 #include "gguf_kernels.hpp"
 #include "gguf_kq_f16.hpp"
+#include "gguf_moe_route.hpp"
 
 namespace gollek {
 
@@ -39,19 +40,18 @@ constexpr int kTailBytes = 64;
 
 }  // namespace
 
-// fp32 rows -> records: rec (row, superblock) 1024 bytes, per half and digit
-// 16 pieces (KqUnit's order, not swizzled); mins 64 bytes; scales one float.
-// A wave takes four rows of one superblock, each row's 16 lanes 16 columns
-// each, and has read them all before it writes (rec may be v itself).
+namespace {
+
+// One row's superblock, fp32 -> record (16 lanes of a wave, 16 columns each):
+// rec (row, superblock) 1024 bytes, per half and digit 16 pieces (KqUnit's
+// order, not swizzled); mins 64 bytes; scales one float.  The lanes have read
+// their columns before they write (rec may be v itself).
 template <int T>
-__global__ __launch_bounds__(256) void moe_records_kernel(const float *v, int rows, int K, uint8_t *rec,
-                                                          uint8_t *__restrict__ mins, float *__restrict__ scales) {
-    const int lane = (int)threadIdx.x & 63, n = lane & 15;
-    const int nsb = K / kQK, sb = (int)blockIdx.x;
-    const int r = 16 * (int)blockIdx.y + (int)(threadIdx.x >> 4);
-    if (r >= rows) return;  // whole rows of 16 lanes
-    const int64_t rs = (int64_t)r * nsb + sb;
-    const f32x4 *const src = reinterpret_cast<const f32x4 *>(v + (int64_t)r * K + kQK * sb + 16 * n);
+__device__ __forceinline__ void record_row(const float *v, int64_t r, int sb, int K, uint8_t *rec,
+                                           uint8_t *__restrict__ mins, float *__restrict__ scales) {
+    const int n = (int)threadIdx.x & 15;
+    const int64_t rs = r * (K / kQK) + sb;
+    const f32x4 *const src = reinterpret_cast<const f32x4 *>(v + r * K + kQK * sb + 16 * n);
     f32x4 x[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) x[i] = src[i];
@@ -86,6 +86,36 @@ __global__ __launch_bounds__(256) void moe_records_kernel(const float *v, int ro
         *reinterpret_cast<uint2 *>(mins + rs * kTailBytes + 16 * (n >> 2) + 8 * ((n >> 1) & 1)) = kq_min_digits(t);
     }
     if (n == 0) scales[rs] = inv;
+}
+
+}  // namespace
+
+// Records of `rows` rows, 16 rows and a superblock a workgroup.
+template <int T>
+__global__ __launch_bounds__(256) void moe_records_kernel(const float *v, int rows, int K, uint8_t *rec,
+                                                          uint8_t *__restrict__ mins, float *__restrict__ scales) {
+    const int r = 16 * (int)blockIdx.y + (int)(threadIdx.x >> 4);
+    if (r < rows) record_row<T>(v, r, (int)blockIdx.x, K, rec, mins, scales);  // whole rows of 16 lanes
+}
+
+// The first launch: workgroup 0 routes, the others build x's records (64 rows'
+// superblocks each), which do not depend on it.  (As two launches 5 us more.)
+template <int T>
+__global__ __launch_bounds__(kRouteThreads) void moe_front_kernel(const int32_t *__restrict__ ids,
+                                                                  const float *__restrict__ wts, int P, int E,
+                                                                  int group, int chunks, int keys_in_lds,
+                                                                  int32_t *__restrict__ meta,
+                                                                  int2 *__restrict__ items, const float *x, int rows,
+                                                                  int K, uint8_t *rec, uint8_t *__restrict__ mins,
+                                                                  float *__restrict__ scales) {
+    extern __shared__ int32_t sh[];
+    if (blockIdx.x == 0) {
+        moe_route(ids, wts, P, E, group, chunks, keys_in_lds, meta, items, sh);
+        return;
+    }
+    const int nsb = K / kQK;
+    const int64_t i = (int64_t)(blockIdx.x - 1) * (kRouteThreads / 16) + (int)(threadIdx.x >> 4);
+    if (i < (int64_t)rows * nsb) record_row<T>(x, i / nsb, (int)(i % nsb), K, rec, mins, scales);
 }
 
 namespace {
@@ -311,9 +341,16 @@ hipError_t launch_moe_gemm(int gate_type, int down_type, const uint8_t *gate, co
     const unsigned items = (unsigned)max_items(P, E, 16 * mt);
     uint8_t *xrec = ws + L.ypair, *hrec = ws + L.h;
     float *h = reinterpret_cast<float *>(hrec), *ypair = reinterpret_cast<float *>(ws + L.ypair);
-    hipError_t e = launch_moe_route(ids, wts, P, E, 16 * mt, meta, list, stream);
-    if (e != hipSuccess) return e;
-    e = launch_records(gate_type, x, T, H, xrec, ws + xt.mins, reinterpret_cast<float *>(ws + xt.scales), stream);
+    const MoeRoutePlan rp = moe_route_plan(P, E);
+    const int64_t xrows = (int64_t)T * (H / kQK);
+    const dim3 fgrid((unsigned)(1 + (xrows + kRouteThreads / 16 - 1) / (kRouteThreads / 16)));
+    auto front = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, fgrid, dim3(kRouteThreads), rp.lds_bytes, stream, ids, wts, P, E, 16 * mt,
+                           rp.chunks, rp.keys_in_lds, meta, list, x, T, H, xrec, ws + xt.mins,
+                           reinterpret_cast<float *>(ws + xt.scales));
+    };
+    gate_type == kQ6_K ? front(&moe_front_kernel<kQ6_K>) : front(&moe_front_kernel<kQ4_K>);
+    hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     e = launch_pass_type<true>(gate_type, mt, items, gate, up, I, H, xrec, ws + xt.mins,
                                reinterpret_cast<const float *>(ws + xt.scales), top_k, list, nitems, offsets, pairs, h,
