@@ -17,8 +17,8 @@
 // What bounds it: a workgroup's stage is short (34 MFMAs a wave at one row
 // tile), so its loads' latency shows; small tiles keep several workgroups on
 // a CU.  128 experts x 768, hidden 2048, Q4_K gate / up, Q6_K down, 256 tokens x
-// top-8: 717 us on the passes of gguf_moe_mfma.hip, 204 here (gate/up 96 us for
-// 226 MB, down 100 us for 165 MB, the other launches 24 us); 32 x 1280,
+// top-8: 717 us on the passes of gguf_moe_mfma.hip, 184 here (the launches beside
+// the two GEMMs 24 us; the weights are 391 MB); 32 x 1280,
 // hidden 2816, 256 tokens x top-4: 2435 us on the row kernels, 157 here.
 //
 // Launches: routing (a list of (expert, first route) items of at most 16 MT
@@ -254,8 +254,6 @@ __global__ __launch_bounds__(64 * NW) void moe_gemm_kernel(const uint8_t *__rest
 
 namespace {
 
-constexpr int kMoeGemmWaves = 4;
-
 // Records' tails and the item list in the workspace's xdig / hdig regions.
 struct RecordTails {
     size_t mins, scales, end;  // byte offsets
@@ -277,20 +275,37 @@ int item_tiles(int64_t P, int E) { return P >= 10 * (int64_t)E ? 2 : 1; }
 
 int64_t max_items(int64_t P, int E, int group) { return (P < E ? P : E) + P / group; }
 
+// Waves of a workgroup.  Eight stage x once for twice the weight rows, but one
+// such workgroup fills a CU: from two rounds over the CUs, by the items to be
+// expected (half a tile more than the routes fill, per expert).  128 x 768, 256
+// tokens x top-8, three rounds: 209 us with four, 194 with eight; 32 x 1280,
+// 100 tokens x top-4, 1.25 rounds: 156 / 184 us.
+bool wide_groups(int64_t P, int E, int mt, int rows_e, int cols) {
+    return (P / (16 * mt) + E / 2) * (rows_e / cols) >= 2 * (int64_t)device_cus();
+}
+
+template <int T, int MT, int NW, bool GATED, class... A>
+hipError_t launch_groups(unsigned items, int rows_e, hipStream_t stream, A... a) {
+    hipLaunchKernelGGL((moe_gemm_kernel<T, MT, NW, GATED>), dim3(items * (unsigned)(rows_e / ((GATED ? 16 : 32) * NW))),
+                       dim3(64 * NW), 0, stream, a...);
+    return hipGetLastError();
+}
+
 template <int T, bool GATED>
-hipError_t launch_pass(int mt, unsigned items, const uint8_t *w0, const uint8_t *w1, int rows_e, int K,
-                       const uint8_t *rec, const uint8_t *mins, const float *scales, int per_record,
+hipError_t launch_pass(int mt, int64_t P, int E, unsigned items, const uint8_t *w0, const uint8_t *w1, int rows_e,
+                       int K, const uint8_t *rec, const uint8_t *mins, const float *scales, int per_record,
                        const int2 *list, const int32_t *nitems, const int32_t *offsets, const int32_t *pairs,
                        float *out, hipStream_t stream) {
-    constexpr int NW = kMoeGemmWaves, cols = (GATED ? 16 : 32) * NW;
-    const dim3 grid(items * (unsigned)(rows_e / cols)), block(64 * NW);
+    auto run = [&](auto launch) {
+        return launch(items, rows_e, stream, w0, w1, rows_e, K, rec, mins, scales, per_record, list, nitems, offsets,
+                      pairs, out);
+    };
+    const bool wide = wide_groups(P, E, mt, rows_e, (GATED ? 16 : 32) * 8);
     if (mt == 1)
-        hipLaunchKernelGGL((moe_gemm_kernel<T, 1, NW, GATED>), grid, block, 0, stream, w0, w1, rows_e, K, rec, mins,
-                           scales, per_record, list, nitems, offsets, pairs, out);
-    else
-        hipLaunchKernelGGL((moe_gemm_kernel<T, 2, NW, GATED>), grid, block, 0, stream, w0, w1, rows_e, K, rec, mins,
-                           scales, per_record, list, nitems, offsets, pairs, out);
-    return hipGetLastError();
+        return wide ? run([](auto... a) { return launch_groups<T, 1, 8, GATED>(a...); })
+                    : run([](auto... a) { return launch_groups<T, 1, 4, GATED>(a...); });
+    return wide ? run([](auto... a) { return launch_groups<T, 2, 8, GATED>(a...); })
+                : run([](auto... a) { return launch_groups<T, 2, 4, GATED>(a...); });
 }
 
 template <bool GATED, class... A>
@@ -352,13 +367,13 @@ hipError_t launch_moe_gemm(int gate_type, int down_type, const uint8_t *gate, co
     gate_type == kQ6_K ? front(&moe_front_kernel<kQ6_K>) : front(&moe_front_kernel<kQ4_K>);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    e = launch_pass_type<true>(gate_type, mt, items, gate, up, I, H, xrec, ws + xt.mins,
+    e = launch_pass_type<true>(gate_type, mt, (int64_t)P, E, items, gate, up, I, H, xrec, ws + xt.mins,
                                reinterpret_cast<const float *>(ws + xt.scales), top_k, list, nitems, offsets, pairs, h,
                                stream);
     if (e != hipSuccess) return e;
     e = launch_records(down_type, h, P, I, hrec, ws + ht.mins, reinterpret_cast<float *>(ws + ht.scales), stream);
     if (e != hipSuccess) return e;
-    e = launch_pass_type<false>(down_type, mt, items, down, down, H, I, hrec, ws + ht.mins,
+    e = launch_pass_type<false>(down_type, mt, (int64_t)P, E, items, down, down, H, I, hrec, ws + ht.mins,
                                 reinterpret_cast<const float *>(ws + ht.scales), 1, list, nitems, offsets, pairs,
                                 ypair, stream);
     if (e != hipSuccess) return e;

@@ -225,6 +225,25 @@ def test_moe_grouped_gemm(gt, dt, E, H, I, c):
         t.close()
 
 
+# Eight-wave workgroups (enough expected items): gate/up of one and two row
+# tiles, down of two; the bound of test_moe_grouped_gemm.
+@pytest.mark.parametrize("gt,dt,E,H,I,T,k", [(syn.Q4_K, syn.Q5_K, 64, 512, 1280, 200, 4),
+                                             (syn.Q5_K, syn.Q6_K, 128, 256, 768, 60, 8),
+                                             (syn.Q6_K, syn.Q4_K, 64, 3072, 256, 200, 4)])
+def test_moe_grouped_gemm_eight_waves(gt, dt, E, H, I, T, k):
+    print(f"[gpu] moe gemm gate={gt} down={dt} E={E} H={H} I={I} T={T} k={k}", flush=True)
+    gate, up, down, tg, tu, td = _experts(E, H, I, seed=E + H, down_type=dt, gate_type=gt)
+    ids, w = syn.moe_routing(T, E, k, seed=61)
+    x = syn.activation(T * H, seed=62).reshape(T, H)
+    out = ops.moe_grouped(tg, tu, td, E, x, ids, w)
+    ref = o.moe_reference_q4k(gate, up, down, E, x, ids, w, down_type=dt, gate_type=gt)
+    err = np.linalg.norm(out.astype(np.float64) - ref) / np.linalg.norm(ref)
+    print(f"[gpu] moe gemm err={err:.3e}", flush=True)
+    assert err <= 2 * 5.7e-6
+    for t in (tg, tu, td):
+        t.close()
+
+
 @pytest.fixture
 def moe_variant():
     def set_variant(v):
