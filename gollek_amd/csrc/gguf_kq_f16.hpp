@@ -283,7 +283,9 @@ __device__ __forceinline__ void static_for(F &&f) {
 // The stage loop: acc[mt][nt] += the contraction of the workgroup's MT row
 // tiles with this wave's two 16-row tiles of W (rows wp[0], wp[1] at lane &
 // 15) over superblocks sb_of(st) of stages [st0, st1).  `units`: the wave's
-// first unit in buffer 0; buffer 1 is `flip` bytes after it.  produce(kc, st,
+// first unit in buffer 0; buffer 1 is `flip` bytes after it.  begin() requests
+// the first stage's x and ready() has it in LDS (the first raw bytes of W are
+// requested between the two, so that their latencies overlap); produce(kc, st,
 // buffer), called in every step of a stage (kc::value = 0 .. 7), brings the x
 // of stage st into that buffer.
 //
@@ -292,10 +294,10 @@ __device__ __forceinline__ void static_for(F &&f) {
 // replace this stage's after their last use, in step 6 (requested a stage
 // ahead into registers of their own they cost the small tiles a workgroup per
 // CU: Q4_K M = 16, 14336 x 4096, 15.0 against 17.7 us).
-template <int T, int MT, int DIGITS, bool CENTERED, class SbOf, class Produce>
+template <int T, int MT, int DIGITS, bool CENTERED, class SbOf, class Begin, class Ready, class Produce>
 __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *const (&wp)[2], const uint8_t *units,
                                           int flip, int st0, int st1, int nsb, int lane, SbOf &&sb_of,
-                                          Produce &&produce) {
+                                          Begin &&begin, Ready &&ready, Produce &&produce) {
     using Op = KqOperand<T, CENTERED>;
     using U = KqUnit<DIGITS>;
     constexpr int NT = Op::kTerms;
@@ -317,7 +319,9 @@ __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *co
             raw[nt].template load_codes<1>(p, g);
         }
     };
+    begin();
     load_w(st0);
+    ready();
     for (int st = st0; st < st1; st++) {
         const int nxt = st + 1 < st1 ? st + 1 : st;
         const uint8_t *const cur = units + ((st - st0) & 1) * flip;

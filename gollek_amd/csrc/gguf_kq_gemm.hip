@@ -13,7 +13,8 @@
 // Against the bf16 kernel with one FMA per 32 columns and output that this
 // replaces: Q4_K M = 2048 456 -> 345 us (697 TFLOP/s), M = 512 134 -> 97;
 // Q6_K M = 333, 4096 x 14336 183 -> 100 us (its scale groups of 16 took three
-// half-empty MFMAs); Q4_K M = 16 19.5 -> 15.4 us.
+// half-empty MFMAs); Q4_K M = 16 19.5 -> 13.9 us (14.9 with the first raw bytes
+// of W requested only once the first x stood in LDS).
 #include "gguf_gemm_plan.hpp"
 #include "gguf_kq_f16.hpp"
 
@@ -120,38 +121,42 @@ __global__ __launch_bounds__(64 * NW *KW, MT == 1 && NW == 2 ? 4 : 1) void gemm_
     int xg, xk0, xk1;
     kq_place<T>(n, xg, xk0, xk1);
     XRows<T> xr[2];
-    auto load_x = [&](int j, int st) {
+    auto load_x = [&](XRows<T> &to, int j, int st) {
         const int q = wave + kWaves * j, u = q >> 2, sb = st * KW + u / MT;
         const int r = m0 + 16 * (u % MT) + 4 * (q & 3) + g;
         // (rows past M repeat row M - 1; their results are not stored)
-        xr[j & 1].load(X + (int64_t)(r < M ? r : M - 1) * K + (int64_t)(sb < nsb ? sb : nsb - 1) * kQK + 16 * n);
+        to.load(X + (int64_t)(r < M ? r : M - 1) * K + (int64_t)(sb < nsb ? sb : nsb - 1) * kQK + 16 * n);
     };
-    auto store_x = [&](int j, int b) {
+    auto store_x = [&](const XRows<T> &from, int j, int b) {
         const int q = wave + kWaves * j, u = q >> 2, lr = 4 * (q & 3) + g;
         uint8_t *const unit = &lds[b][u * U::kBytes];
-        xr[j & 1].store(unit + U::piece(xk0, xg, lr), unit + U::piece(xk1, xg, lr),
+        from.store(unit + U::piece(xk0, xg, lr), unit + U::piece(xk1, xg, lr),
                         unit + U::kMins + 64 * lr + 16 * (n >> 2) + 8 * ((n >> 1) & 1),
                         reinterpret_cast<float *>(unit + U::kScales) + lr, lane);
     };
-    load_x(0, st0);
+    XRows<T> first[kPer];
+    kq_stages<T, MT, 1, false>(
+        acc, wp, &lds[0][kw * MT * U::kBytes], UN * U::kBytes, st0, st1, nsb, lane, sb_of,
+        [&] {
 #pragma unroll
-    for (int j = 0; j < kPer; j++) {
-        if (j + 1 < kPer) load_x(j + 1, st0);
-        store_x(j, 0);
-    }
-    __syncthreads();
-    kq_stages<T, MT, 1, false>(acc, wp, &lds[0][kw * MT * U::kBytes], UN * U::kBytes, st0, st1, nsb, lane, sb_of,
-                        [&](auto kc, int st, int b) {
-                            constexpr int k = kc.value;
-                            if (k == 0) load_x(0, st);
-                            if (k == 0 && kPer > 1) load_x(1, st);
-                            if (k == 3) store_x(0, b);
-                            if (k == 3 && kPer > 2) load_x(2, st);
-                            if (k == 4 && kPer > 1) store_x(1, b);
-                            if (k == 4 && kPer > 3) load_x(3, st);
-                            if (k == 6 && kPer > 2) store_x(2, b);
-                            if (k == 7 && kPer > 3) store_x(3, b);
-                        });
+            for (int j = 0; j < kPer; j++) load_x(first[j], j, st0);
+        },
+        [&] {
+#pragma unroll
+            for (int j = 0; j < kPer; j++) store_x(first[j], j, 0);
+            __syncthreads();
+        },
+        [&](auto kc, int st, int b) {
+            constexpr int k = kc.value;
+            if (k == 0) load_x(xr[0], 0, st);
+            if (k == 0 && kPer > 1) load_x(xr[1], 1, st);
+            if (k == 3) store_x(xr[0], 0, b);
+            if (k == 3 && kPer > 2) load_x(xr[0], 2, st);
+            if (k == 4 && kPer > 1) store_x(xr[1], 1, b);
+            if (k == 4 && kPer > 3) load_x(xr[1], 3, st);
+            if (k == 6 && kPer > 2) store_x(xr[0], 2, b);
+            if (k == 7 && kPer > 3) store_x(xr[1], 3, b);
+        });
 
     if constexpr (KW > 1) {
         f32x4 *const red = reinterpret_cast<f32x4 *>(lds[0]);

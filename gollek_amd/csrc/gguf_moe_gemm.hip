@@ -170,15 +170,18 @@ __device__ __forceinline__ void moe_item(const uint8_t *const (&wp)[2], int nsb,
         if (tid < 16 * MT)
             *reinterpret_cast<float *>(lds + (b * MT + (tid >> 4)) * U::kBytes + U::kScales + 4 * (tid & 15)) = sc;
     };
-    load_tail(0);
-#pragma unroll
-    for (int bt = 0; bt < kBatches; bt++) {
-        load(bt, 0);
-        store(bt, 0);
-    }
-    store_tail(0);
-    __syncthreads();
     kq_stages<T, MT, 2, true>(acc, wp, lds, MT * U::kBytes, 0, nsb, nsb, lane, [](int st) { return st; },
+                        [&] {  // (requesting W before x is in LDS changed nothing here)
+                            load_tail(0);
+#pragma unroll
+                            for (int bt = 0; bt < kBatches; bt++) {
+                                load(bt, 0);
+                                store(bt, 0);
+                            }
+                            store_tail(0);
+                            __syncthreads();
+                        },
+                        [] {},
                         [&](auto kc, int sb, int b) {
                             constexpr int k = kc.value, per = 8 / kBatches;
                             if constexpr (k == 0) load_tail(sb);
