@@ -729,7 +729,7 @@ hipError_t launch_expert(int nsb, const uint8_t *w0, const uint8_t *w1, int64_t 
 
 hipError_t launch_moe_route(const int32_t *ids, const float *wts, int P, int E, int32_t *meta, hipStream_t stream) {
     const MoeRoutePlan p = moe_route_plan(P, E);
-    hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(kRouteThreads), p.lds_bytes, stream, ids, wts, P, E, p.chunks,
+    hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(p.threads), p.lds_bytes, stream, ids, wts, P, E, p.chunks,
                        p.keys_in_lds, meta);
     return hipGetLastError();
 }

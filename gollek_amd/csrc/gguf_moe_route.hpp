@@ -8,16 +8,19 @@ namespace gollek {
 
 constexpr int kRouteThreads = 1024;
 
-// Launch parameters of the routing: 16 chunks while their counters fit 32 KB,
-// and the routes' keys in LDS for the scatter while everything fits the
-// default 64 KB (it otherwise reloads them, one round trip per 64).
+// Launch parameters of the routing: a chunk a wave of the workgroup while their
+// counters fit 32 KB (one for few routes, whose serial scatter is shorter than
+// the larger workgroup's start), and the routes' keys in LDS for the scatter
+// while everything fits the default 64 KB (it otherwise reloads them, one
+// round trip per 64).
 struct MoeRoutePlan {
-    int chunks, keys_in_lds;
+    int threads, chunks, keys_in_lds;
     size_t lds_bytes;
 };
 inline MoeRoutePlan moe_route_plan(int P, int E) {
     MoeRoutePlan p;
-    p.chunks = 16 * (size_t)E * sizeof(int32_t) <= 32768 ? 16 : 1;
+    p.threads = P <= 512 ? 256 : kRouteThreads;
+    p.chunks = P > 512 && 16 * (size_t)E * sizeof(int32_t) <= 32768 ? 16 : 1;
     const size_t base = (size_t)(1 + p.chunks) * (size_t)E * sizeof(int32_t);
     p.keys_in_lds = base + (size_t)P * sizeof(int32_t) <= 65536 ? 1 : 0;
     p.lds_bytes = base + (p.keys_in_lds ? (size_t)P * sizeof(int32_t) : 0);
@@ -33,7 +36,7 @@ inline MoeRoutePlan moe_route_plan(int P, int E) {
 // The routes are cut into `chunks` runs, one a wave (1: all of them in wave
 // 0's scatter): each counts its own keys, so the scatters run side by side
 // (2048 routes: 23 us in one wave, 6.6 us in 16).
-// Called by all kRouteThreads threads of the workgroup; sh: the plan's LDS
+// Called by all threads of the workgroup (at least 64 a chunk); sh: the plan's LDS
 // bytes, cnt[E], run[chunks][E], then (keys_in_lds) key[P].
 __device__ inline void moe_route(const int32_t *__restrict__ ids, const float *__restrict__ wts, int P, int E,
                                  int group, int chunks, int keys_in_lds, int32_t *__restrict__ meta,
@@ -44,16 +47,16 @@ __device__ inline void moe_route(const int32_t *__restrict__ ids, const float *_
     int32_t *nitems = nused + 1;
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int per = ((P + chunks - 1) / chunks + 63) / 64 * 64;  // routes of a chunk
-    for (int i = tid; i < chunks * E; i += kRouteThreads) run[i] = 0;
+    for (int i = tid; i < chunks * E; i += (int)blockDim.x) run[i] = 0;
     __syncthreads();
-    for (int p = tid; p < P; p += kRouteThreads) {
+    for (int p = tid; p < P; p += (int)blockDim.x) {
         const int e = ids[p];
         const bool valid = e >= 0 && e < E && wts[p] != 0.0f;
         if (valid) atomicAdd(&run[p / per * E + e], 1);  // LDS atomic
         if (keys_in_lds) keys[p] = valid ? e : -1;
     }
     __syncthreads();
-    for (int e = tid; e < E; e += kRouteThreads) {
+    for (int e = tid; e < E; e += (int)blockDim.x) {
         int c = 0;
         for (int k = 0; k < chunks; k++) {
             const int n = run[k * E + e];
