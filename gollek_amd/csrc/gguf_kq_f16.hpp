@@ -25,6 +25,7 @@
 // each (A) against m_2g, m_2g+1 three times each (B).
 #pragma once
 
+#include <type_traits>
 #include <utility>
 
 #include "gguf_blocks.hpp"
@@ -286,14 +287,17 @@ __device__ __forceinline__ void static_for(F &&f) {
 // first unit in buffer 0; buffer 1 is `flip` bytes after it.  begin() requests
 // the first stage's x and ready() has it in LDS (the first raw bytes of W are
 // requested between the two, so that their latencies overlap); produce(kc, st,
-// buffer), called in every step of a stage (kc::value = 0 .. 7), brings the x
-// of stage st into that buffer.
+// buffer), called in every step (kc::value = 0 .. 7) of a stage that another one
+// follows, brings the x of stage st into that buffer.
 //
 // A step takes 2 MT DIGITS kTerms MFMAs (one fragment of W); the next
 // fragment's codes are widened while they run.  The next stage's raw bytes
 // replace this stage's after their last use, in step 6 (requested a stage
 // ahead into registers of their own they cost the small tiles a workgroup per
-// CU: Q4_K M = 16, 14336 x 4096, 15.0 against 17.7 us).
+// CU: Q4_K M = 16, 14336 x 4096, 15.0 against 17.7 us).  The last stage is a copy
+// of its own without either: brought in again for nobody, they cost a wait for
+// x and a conversion (Q5_K M = 5, 1024 x 2048, one stage of eight slices: 8.44
+// against 7.19 us; Q6_K M = 333, 4096 x 14336: 101.4 against 98.6).
 template <int T, int MT, int DIGITS, bool CENTERED, class SbOf, class Begin, class Ready, class Produce>
 __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *const (&wp)[2], const uint8_t *units,
                                           int flip, int st0, int st1, int nsb, int lane, SbOf &&sb_of,
@@ -322,8 +326,7 @@ __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *co
     begin();
     load_w(st0);
     ready();
-    for (int st = st0; st < st1; st++) {
-        const int nxt = st + 1 < st1 ? st + 1 : st;
+    auto stage = [&](int st, auto last) {
         const uint8_t *const cur = units + ((st - st0) & 1) * flip;
         f32x4 p[MT][2];
         Op op[2];
@@ -357,9 +360,9 @@ __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *co
                     if constexpr (hc.value == 0) op[0].frag(raw[0], g, kq_order<T>(k + 1), b[(k + 1) & 1][0]);
                     if constexpr (hc.value == R - 1) op[1].frag(raw[1], g, kq_order<T>(k + 1), b[(k + 1) & 1][1]);
                 }
-                if constexpr (hc.value == DIGITS * HN - 1) {
-                    if constexpr (k == 6) load_w(nxt);
-                    produce(kc, nxt, (st + 1 - st0) & 1);
+                if constexpr (hc.value == DIGITS * HN - 1 && !last.value) {
+                    if constexpr (k == 6) load_w(st + 1);
+                    produce(kc, st + 1, (st + 1 - st0) & 1);
                 }
                 // fragment reads, then the widening and conversion between the MFMAs
                 __builtin_amdgcn_sched_group_barrier(0x100, MH, 0);
@@ -401,7 +404,9 @@ __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *co
                 }
         }
         __syncthreads();
-    }
+    };
+    for (int st = st0; st < st1 - 1; st++) stage(st, std::false_type{});
+    stage(st1 - 1, std::true_type{});
 }
 
 }  // namespace kqf
