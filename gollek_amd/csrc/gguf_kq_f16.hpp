@@ -11,8 +11,12 @@
 // FMA per 32-element block, four VALU instructions per MFMA).
 //
 // x: each (row, superblock) is scaled by a power of two that brings its
-// largest magnitude to [2^8, 2^9); bf16 elements are then exact in fp16 unless
-// they are below 2^-23 of that maximum, where the error is below 2^-33 of it.
+// largest magnitude to [2^14, 2^15); bf16 elements are then exact in fp16
+// unless they are below 2^-31 of that maximum, where the error is at most 2^-39
+// of it.  Rows with an outlier of 2^20 times some 16 columns' largest and more
+// (kq_wide), and those with an infinity (the parts of a Q6_K product would cancel
+// to NaN), are computed again by kq_wide_rows (Q4_K M = 512, 14336 x 4096: 229 us
+// with one such row, 1030 with 512 of them, 104 with none on the same card).
 //
 // Column order.  Which 8 columns of the superblock lane group g (lane >> 4)
 // supplies to MFMA i is free as long as both operands agree, so it follows
@@ -21,8 +25,9 @@
 // with one AND each.
 //
 // Min term (Q4_K, Q5_K): sum_j m_j * sum(x of sub-block j) is one more MFMA:
-// lane group g holds the sums of sub-blocks 2g, 2g + 1 as three fp16 digits
-// each (A) against m_2g, m_2g+1 three times each (B).
+// lane group g holds the sums of sub-blocks 2g, 2g + 1 (up to 2^20, as 2^-6 of
+// that) as three fp16 digits each (A), the second and third times 2^12, against
+// m_2g, m_2g+1 once and twice times 2^-12 (B).
 #pragma once
 
 #include <type_traits>
@@ -131,6 +136,14 @@ __device__ __forceinline__ f16x8 as_h8(const uint32_t (&v)[4]) {
 }
 __device__ __forceinline__ f16x2 splat(_Float16 v) { return f16x2{v, v}; }
 
+// Two codes (bytes 0 and 1 of w) against kq_min_digits: v, v 2^-12, v 2^-12
+// each (an integer v is the fp16 subnormal v 2^-24).
+__device__ __forceinline__ f16x8 kq_digit_codes(uint32_t w) {
+    const f16x2 b = as_h2((w & 0xFFu) | (w >> 8) << 16) * splat((_Float16)0x1p12f), a = b * splat((_Float16)0x1p12f);
+    const _Float16 z = (_Float16)0.0f;
+    return f16x8{a[0], b[0], b[0], z, a[1], b[1], b[1], z};
+}
+
 // One 16-row tile's operand of a superblock.  head() decodes the row's scale
 // codes, the min operand and the fp32 factors; frag() the codes of one MFMA
 // (kTerms operands) from the raw bytes.
@@ -168,16 +181,12 @@ struct KqOperand {
             q4k_pair_codes(r.hd.y, r.hd.z, r.hd.w, g, &scp, &mnp);
             s[0] = splat((_Float16)(unsigned short)((scp & 0xFFu) << 9));
             s[1] = splat((_Float16)(unsigned short)((scp >> 8) << 5));
-            const _Float16 m0 = (_Float16)(unsigned short)(mnp & 0xFFu), m1 = (_Float16)(unsigned short)(mnp >> 8);
-            bm = f16x8{m0, m0, m0, (_Float16)0.0f, m1, m1, m1, (_Float16)0.0f};
-            if constexpr (kCentered) {
-                const _Float16 c0 = (_Float16)(unsigned short)(scp & 0xFFu), c1 = (_Float16)(unsigned short)(scp >> 8);
-                bs = f16x8{c0, c0, c0, (_Float16)0.0f, c1, c1, c1, (_Float16)0.0f};
-            }
+            bm = kq_digit_codes(mnp);
+            if constexpr (kCentered) bs = kq_digit_codes(scp);
             d = half_bits_to_float_fast(r.hd.x & 0xFFFFu) * kq_code_scale<T>();
             // no min code set: a non-finite dmin stays out
             // (RT/GgufKQuantLayout.java:67-69)
-            dm = (r.hd.z | (r.hd.w & 0xF0F0F0F0u)) != 0u ? half_bits_to_float_fast(r.hd.x >> 16) : 0.0f;
+            dm = (r.hd.z | (r.hd.w & 0xF0F0F0F0u)) != 0u ? half_bits_to_float_fast(r.hd.x >> 16) * 0x1p6f : 0.0f;
         }
     }
     __device__ __forceinline__ void frag(const KqRaw<T> &r, int g, int i, f16x8 (&b)[kTerms]) const {
@@ -254,19 +263,32 @@ __device__ __forceinline__ float row_max16(float v) {
     return fmaxf(v, kq_dpp<0x128>(v));  // row_ror:8
 }
 
-// max |v| < 2^(E - 126) (E: biased exponent of the largest magnitude): the
-// power of two that brings it to [2^8, 2^9), and its inverse.
+// For a row's superblock whose largest magnitude is mx: the power of two that
+// brings it to [2^14, 2^15), and its inverse (magnitudes below 2^-106 are scaled
+// as that one, so that kq_wide's bound is a normal number).
 __device__ __forceinline__ void kq_row_scale(float mx, float &s, float &inv) {
-    uint32_t e = (__float_as_uint(mx) >> 23) & 0xFFu;
-    e = e < 9u ? 9u : e;
-    s = __uint_as_float((262u - e) << 23);
-    inv = __uint_as_float((e - 8u) << 23);
+    uint32_t e = __float_as_uint(mx) & 0x7F800000u;
+    e = e < (21u << 23) ? 21u << 23 : e;
+    s = __uint_as_float((268u << 23) - e);
+    inv = __uint_as_float(e - (14u << 23));
 }
 
-// t (|t| <= 2^14) as three fp16 digits (half of a lane's slots of KqOperand::bm).
+// Whether a row's superblock of maximum `mx` is one for kq_wide_rows, by 16 of
+// its columns, of maximum `lane_mx`: an infinity, or 16 that are not all zero
+// and below 2^-6 when scaled, where fp16's rounding is 2^-19 of their largest (an
+// outlier of 2^20 times the rest, its weights 0: 1.5e-7 of error in the result,
+// fp32 sums of K = 2048 1 to 6e-7).  The lanes that find it so (a ballot each: of
+// the two together it takes a select and a second comparison).
+__device__ __forceinline__ uint64_t kq_wide(float lane_mx, float mx, float inv) {
+    return __builtin_amdgcn_ballot_w64(__float_as_uint(lane_mx) - 1u < __float_as_uint(inv) - (6u << 23)) |
+           __builtin_amdgcn_ballot_w64(mx == __builtin_inff());
+}
+
+// t (|t| <= 2^14) as three fp16 digits, the second and third times 2^12 (half of
+// a lane's slots of KqOperand::bm).
 __device__ __forceinline__ uint2 kq_min_digits(float t) {
     const _Float16 a = (_Float16)t;
-    const float r = t - (float)a;
+    const float r = (t - (float)a) * 0x1p12f;
     const _Float16 b = (_Float16)r;
     const _Float16 c = (_Float16)(r - (float)b);
     return uint2{as_u(f16x2{a, b}), as_u(f16x2{c, (_Float16)0.0f})};
@@ -283,12 +305,15 @@ __device__ __forceinline__ void static_for(F &&f) {
 
 // The stage loop: acc[mt][nt] += the contraction of the workgroup's MT row
 // tiles with this wave's two 16-row tiles of W (rows wp[0], wp[1] at lane &
-// 15) over superblocks sb_of(st) of stages [st0, st1).  `units`: the wave's
-// first unit in buffer 0; buffer 1 is `flip` bytes after it.  begin() requests
-// the first stage's x and ready() has it in LDS (the first raw bytes of W are
-// requested between the two, so that their latencies overlap); produce(kc, st,
-// buffer), called in every step (kc::value = 0 .. 7) of a stage that another one
-// follows, brings the x of stage st into that buffer.
+// 15) over superblocks sb_of(st) of stages [st0, st1) (WHOLE: none is past the
+// last; otherwise selects, 64 of the 870 VALU instructions of a 128-row stage,
+// keep those out).  `units`: the wave's first unit in buffer 0; buffer 1 is `flip`
+// bytes after it.  begin() requests the first stage's x and ready() has it in LDS
+// (the first raw bytes of W are requested between the two, so that their
+// latencies overlap); produce(kc, st, buffer), called in every step (kc::value =
+// 0 .. 7) of a stage that another one follows, brings the x of stage st into that
+// buffer; done() runs before the last stage, whose barrier publishes what it
+// writes to LDS.
 //
 // A step takes 2 MT DIGITS kTerms MFMAs (one fragment of W); the next
 // fragment's codes are widened while they run.  The next stage's raw bytes
@@ -298,10 +323,10 @@ __device__ __forceinline__ void static_for(F &&f) {
 // of its own without either: brought in again for nobody, they cost a wait for
 // x and a conversion (Q5_K M = 5, 1024 x 2048, one stage of eight slices: 8.44
 // against 7.19 us; Q6_K M = 333, 4096 x 14336: 101.4 against 98.6).
-template <int T, int MT, int DIGITS, bool CENTERED, class SbOf, class Begin, class Ready, class Produce>
+template <int T, int MT, int DIGITS, bool CENTERED, bool WHOLE, class SbOf, class Begin, class Ready, class Produce, class Done>
 __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *const (&wp)[2], const uint8_t *units,
                                           int flip, int st0, int st1, int nsb, int lane, SbOf &&sb_of,
-                                          Begin &&begin, Ready &&ready, Produce &&produce) {
+                                          Begin &&begin, Ready &&ready, Produce &&produce, Done &&done) {
     using Op = KqOperand<T, CENTERED>;
     using U = KqUnit<DIGITS>;
     constexpr int NT = Op::kTerms;
@@ -336,7 +361,7 @@ __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *co
             op[nt].head(raw[nt], g);
             op[nt].frag(raw[nt], g, kq_order<T>(0), b[0][nt]);
         }
-        const bool act = sb_of(st) < nsb;  // uniform
+        const bool act = WHOLE || sb_of(st) < nsb;  // uniform
         static_for<8>([&](auto kc) {
             constexpr int k = kc.value;
             static_for<DIGITS * HN>([&](auto hc) {
@@ -392,8 +417,8 @@ __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *co
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     float v = p[mt][nt][r];
-                    if constexpr (Op::kCentered) {  // d P + (d 2^-15 8 PS - dmin PM): the small part last
-                        const float c = op[nt].d * (T == kQ5_K ? 0x1p-11f : 0x1p-12f);
+                    if constexpr (Op::kCentered) {  // d P + (d 2^-15 8 PS 2^6 - dmin PM 2^6): the small part last
+                        const float c = op[nt].d * (T == kQ5_K ? 0x1p-5f : 0x1p-6f);
                         v = fmaf(op[nt].d, v, fmaf(c, ps[nt][r], -op[nt].dm * pm[nt][r]));
                     } else {
                         v *= op[nt].d;
@@ -406,7 +431,75 @@ __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *co
         __syncthreads();
     };
     for (int st = st0; st < st1 - 1; st++) stage(st, std::false_type{});
+    done();
     stage(st1 - 1, std::true_type{});
+}
+
+// acc of the rows whose bit is set in `wide` (16 MT bits, the same in all waves),
+// over the stages that kq_stages contracted, from dequantized weights on the fp32
+// matrix cores, whole row tiles at a time.  Lane group g takes 64 columns of a
+// superblock, of x and W alike: load_x(row, superblock, c, v) columns 16 c .. + 15
+// of a row of the tile, and W's as its raw bytes stand.  Seldom called, so its
+// loops are left rolled: it has to fit the registers that the stages leave.
+template <int T, int MT, class SbOf, class LoadX>
+__device__ __forceinline__ void kq_wide_rows(const uint32_t *wide, f32x4 (&acc)[MT][2], const uint8_t *const (&wp)[2],
+                                             int st0, int st1, int nsb, int lane, SbOf &&sb_of, LoadX &&load_x) {
+    const int g = lane >> 4, n = lane & 15;
+#pragma unroll 1
+    for (int mt = 0; mt < MT; mt++) {
+        const uint32_t bits = (uint32_t)__builtin_amdgcn_readfirstlane((int)((wide[mt >> 1] >> (16 * (mt & 1))) & 0xFFFFu));
+        if (bits == 0u) continue;
+        f32x4 y[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll 1
+        for (int st = st0; st < st1; st++) {
+            const int sb = sb_of(st);
+            if (sb >= nsb) break;
+#pragma unroll 1
+            for (int t = 0; t < 4; t++) {  // 16 columns: nibble t >> 1 of byte run t & 1
+                float v[16];
+                load_x(16 * mt + n, sb, T == kQ6_K ? 8 * (g >> 1) + 2 * t + (g & 1) : 4 * g + t, v);
+#pragma unroll
+                for (int nt = 0; nt < 2; nt++) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    f32x4 part = {0.0f, 0.0f, 0.0f, 0.0f};  // (one running sum has four times the error)
+                    const uint8_t *const p = wp[nt] + (int64_t)sb * kq_block_bytes<T>();
+                    KqRaw<T> r;
+                    r.load_head(p, g);
+                    r.template load_codes<0>(p, g);
+                    r.template load_codes<1>(p, g);
+                    float s, m = 0.0f;  // the 16 columns' d sc and dmin m
+                    if constexpr (T == kQ6_K) {
+                        const uint32_t w = (t & 2) ? r.s1 : r.s0;
+                        s = half_bits_to_float_fast(r.d) * (float)(int8_t)(w >> (16 * (t & 1) + 8 * (g & 1)));
+                    } else {
+                        uint32_t scp, mnp;
+                        q4k_pair_codes(r.hd.y, r.hd.z, r.hd.w, g, &scp, &mnp);
+                        const uint32_t mc = (mnp >> (8 * (t >> 1))) & 0xFFu;
+                        s = half_bits_to_float_fast(r.hd.x & 0xFFFFu) * (float)((scp >> (8 * (t >> 1))) & 0xFFu);
+                        m = mc ? half_bits_to_float_fast(r.hd.x >> 16) * (float)mc : 0.0f;
+                    }
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        const int k = i >> 2, at = 8 * (i & 3);
+                        int q = (int)((((t & 1) ? r.q1[k] : r.q0[k]) >> (at + 4 * (t >> 1))) & 15u);
+                        if constexpr (T == kQ5_K)
+                            q |= (int)((((t & 1) ? r.h1[k] : r.h0[k]) >> (at + 2 * g + (t >> 1))) & 1u) << 4;
+                        if constexpr (T == kQ6_K) q = (q | (int)((r.h0[k] >> (at + 2 * t)) & 3u) << 4) - 32;
+                        part = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i], s * (float)q - m, part, 0, 0, 0);
+                    }
+                    y[nt] += part;
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < MT; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (j == mt && ((bits >> (4 * g + r)) & 1u) != 0u) {
+                    acc[j][0][r] = y[0][r];
+                    acc[j][1][r] = y[1][r];
+                }
+    }
 }
 
 }  // namespace kqf

@@ -35,8 +35,9 @@ struct XRows {
         x[0] = *reinterpret_cast<const v4u *>(p);
         x[1] = *reinterpret_cast<const v4u *>(p + 8);
     }
-    // p0, p1: the lane's two pieces, mins: its sub-block's half of a min piece
-    __device__ __forceinline__ void store(uint8_t *p0, uint8_t *p1, uint8_t *mins, float *scale, int lane) const {
+    // p0, p1: the lane's two pieces, mins: its sub-block's half of a min piece;
+    // returns the lanes that find their row a wide one
+    __device__ __forceinline__ uint64_t store(uint8_t *p0, uint8_t *p1, uint8_t *mins, float *scale, int lane) const {
         float v[16], mx = 0.0f;
 #pragma unroll
         for (int i = 0; i < 16; i++) {
@@ -45,6 +46,7 @@ struct XRows {
         }
 #pragma unroll
         for (int i = 0; i < 16; i += 2) mx = fmaxf(fmaxf(mx, fabsf(v[i])), fabsf(v[i + 1]));
+        const float lane_mx = mx;
         mx = row_max16(mx);
         float s, inv, t = 0.0f;
         kq_row_scale(mx, s, inv);
@@ -56,7 +58,7 @@ struct XRows {
                 const int e = 8 * h + 4 * (j >> 1) + (j & 1);
                 const f16x2 c = {(_Float16)(v[e] * s), (_Float16)(v[e + 2] * s)};
                 f[j] = as_u(c);
-                if constexpr (KqOperand<T, false>::kMins) t = __builtin_amdgcn_fdot2(c, splat((_Float16)1.0f), t, false);
+                if constexpr (KqOperand<T, false>::kMins) t = __builtin_amdgcn_fdot2(c, splat((_Float16)0x1p-6f), t, false);
             }
             *reinterpret_cast<f16x8 *>(h ? p1 : p0) = as_h8(f);
         }
@@ -65,6 +67,7 @@ struct XRows {
             *reinterpret_cast<uint2 *>(mins) = kq_min_digits(t);  // both lanes write the same 8 bytes
         }
         if ((lane & 15) == 0) *scale = inv;
+        return kq_wide(lane_mx, mx, inv);
     }
 };
 
@@ -81,7 +84,9 @@ __global__ __launch_bounds__(64 * NW *KW, MT == 1 && NW == 2 ? 4 : 1) void gemm_
     constexpr int kTileM = 16 * MT, kTileN = 32 * NW;
     using U = KqUnit<1>;
     __shared__ __attribute__((aligned(16))) uint8_t lds[2][UN * U::kBytes];
+    __shared__ uint32_t wide[(kTileM + 31) / 32];  // the tile's rows for kq_wide_rows
 
+    if (threadIdx.x < (kTileM + 31) / 32) wide[threadIdx.x] = 0u;
     const int lane = (int)threadIdx.x & 63, n = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int nw = wave % NW, kw = wave / NW;
@@ -121,6 +126,7 @@ __global__ __launch_bounds__(64 * NW *KW, MT == 1 && NW == 2 ? 4 : 1) void gemm_
     int xg, xk0, xk1;
     kq_place<T>(n, xg, xk0, xk1);
     XRows<T> xr[2];
+    uint64_t found[kPer] = {};
     auto load_x = [&](XRows<T> &to, int j, int st) {
         const int q = wave + kWaves * j, u = q >> 2, sb = st * KW + u / MT;
         const int r = m0 + 16 * (u % MT) + 4 * (q & 3) + g;
@@ -130,12 +136,12 @@ __global__ __launch_bounds__(64 * NW *KW, MT == 1 && NW == 2 ? 4 : 1) void gemm_
     auto store_x = [&](const XRows<T> &from, int j, int b) {
         const int q = wave + kWaves * j, u = q >> 2, lr = 4 * (q & 3) + g;
         uint8_t *const unit = &lds[b][u * U::kBytes];
-        from.store(unit + U::piece(xk0, xg, lr), unit + U::piece(xk1, xg, lr),
-                        unit + U::kMins + 64 * lr + 16 * (n >> 2) + 8 * ((n >> 1) & 1),
-                        reinterpret_cast<float *>(unit + U::kScales) + lr, lane);
+        found[j] |= from.store(unit + U::piece(xk0, xg, lr), unit + U::piece(xk1, xg, lr),
+                               unit + U::kMins + 64 * lr + 16 * (n >> 2) + 8 * ((n >> 1) & 1),
+                               reinterpret_cast<float *>(unit + U::kScales) + lr, lane);
     };
     XRows<T> first[kPer];
-    kq_stages<T, MT, 1, false>(
+    kq_stages<T, MT, 1, false, KW == 1>(
         acc, wp, &lds[0][kw * MT * U::kBytes], UN * U::kBytes, st0, st1, nsb, lane, sb_of,
         [&] {
 #pragma unroll
@@ -156,6 +162,32 @@ __global__ __launch_bounds__(64 * NW *KW, MT == 1 && NW == 2 ? 4 : 1) void gemm_
             if (k == 4 && kPer > 3) load_x(xr[1], 3, st);
             if (k == 6 && kPer > 2) store_x(xr[0], 2, b);
             if (k == 7 && kPer > 3) store_x(xr[1], 3, b);
+        },
+        [&] {
+#pragma unroll
+            for (int j = 0; j < kPer; j++) {
+                const int q = wave + kWaves * j, row = 16 * ((q >> 2) % MT) + 4 * (q & 3);
+                if (found[j] == 0u) continue;
+                uint32_t rows = 0u;
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    rows |= ((found[j] >> (16 * i)) & 0xFFFFu) != 0u && m0 + row + i < M ? 1u << i : 0u;
+                if (lane == 0) atomicOr(&wide[row >> 5], rows << (row & 31));  // LDS atomic
+            }
+        });
+    uint32_t any = 0u;
+#pragma unroll
+    for (int i = 0; i < (kTileM + 31) / 32; i++) any |= wide[i];
+    if (__builtin_amdgcn_readfirstlane((int)any) != 0)
+        kq_wide_rows<T, MT>(wide, acc, wp, st0, st1, nsb, lane, sb_of, [&](int row, int sb, int c, float (&v)[16]) {
+            const int r = m0 + row;
+            const v4u *const p = reinterpret_cast<const v4u *>(X + (int64_t)(r < M ? r : M - 1) * K + (int64_t)sb * kQK + 16 * c);
+            const v4u a = p[0], b = p[1];
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const uint32_t w = (i < 8 ? a : b)[(i >> 1) & 3];
+                v[i] = __uint_as_float((i & 1) ? w & 0xFFFF0000u : w << 16);
+            }
         });
 
     if constexpr (KW > 1) {

@@ -8,11 +8,16 @@
 // of them instead of once per four routes.
 //
 // fp32 vectors are two fp16 digits: with a row's superblock scaled to a
-// maximum in [2^8, 2^9), v = hi + lo leaves an error below 2^-23 of v or 2^-33
-// of the maximum (the passes this replaces keep 2^-22 of it); both digits
+// maximum in [2^14, 2^15), v = hi + lo leaves an error below 2^-23 of v or 2^-39
+// of the maximum (the two-launch passes keep 2^-22 of it; against the fp32 row
+// kernels the roundings of the products weigh more: 4.5e-7 of error against
+// 7e-7); both digits
 // contract against the same exact weight operand into one fp32 accumulator.
 // They are built once per vector ("records") by a kernel of its own, x's into
 // the workspace's ypair region (free until the down pass), h's in place.
+// Superblocks of too wide a range and those with an infinity (kq_wide) stay
+// fp32, marked by a negative scale, and the rows that hold one are computed
+// again from the packed weights.
 //
 // What bounds it: a workgroup's stage is short (34 MFMAs a wave at one row
 // tile), so its loads' latency shows; small tiles keep several workgroups on
@@ -44,8 +49,9 @@ namespace {
 
 // One row's superblock, fp32 -> record (16 lanes of a wave, 16 columns each):
 // rec (row, superblock) 1024 bytes, per half and digit 16 pieces (KqUnit's
-// order, not swizzled); mins 64 bytes; scales one float.  The lanes have read
-// their columns before they write (rec may be v itself).
+// order, not swizzled); mins 64 bytes; scales one float.  A wide superblock's
+// rec is its 256 floats and its scale negative (mins not written).  The lanes
+// have read their columns before they write (rec may be v itself).
 template <int T>
 __device__ __forceinline__ void record_row(const float *v, int64_t r, int sb, int K, uint8_t *rec,
                                            uint8_t *__restrict__ mins, float *__restrict__ scales) {
@@ -58,12 +64,20 @@ __device__ __forceinline__ void record_row(const float *v, int64_t r, int sb, in
     float mx = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; i++) mx = fmaxf(mx, fabsf(x[i >> 2][i & 3]));
+    const float lane_mx = mx;
     mx = row_max16(mx);
     float s, inv, t = 0.0f;
     kq_row_scale(mx, s, inv);
+    uint8_t *const dst = rec + rs * 1024;
+    const uint64_t found = kq_wide(lane_mx, mx, inv);
+    if (((found >> (threadIdx.x & 48u)) & 0xFFFFu) != 0u) {  // the row's 16 lanes alike
+#pragma unroll
+        for (int i = 0; i < 4; i++) reinterpret_cast<f32x4 *>(dst + 64 * n)[i] = x[i];
+        if (n == 0) scales[rs] = -inv;
+        return;
+    }
     int g, kk[2];
     kq_place<T>(n, g, kk[0], kk[1]);
-    uint8_t *const dst = rec + rs * 1024;
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         uint32_t f[2][4];
@@ -83,7 +97,8 @@ __device__ __forceinline__ void record_row(const float *v, int64_t r, int sb, in
     }
     if constexpr (KqOperand<T, true>::kMins) {
         t += kq_dpp<0xB1>(t);  // the sub-block's other 16 columns
-        *reinterpret_cast<uint2 *>(mins + rs * kTailBytes + 16 * (n >> 2) + 8 * ((n >> 1) & 1)) = kq_min_digits(t);
+        *reinterpret_cast<uint2 *>(mins + rs * kTailBytes + 16 * (n >> 2) + 8 * ((n >> 1) & 1)) =
+            kq_min_digits(t * 0x1p-6f);
     }
     if (n == 0) scales[rs] = inv;
 }
@@ -120,12 +135,39 @@ __global__ __launch_bounds__(kRouteThreads) void moe_front_kernel(const int32_t 
 
 namespace {
 
+// Columns 16 c .. + 15 of a record.
+template <int T>
+__device__ __forceinline__ void record_columns(const uint8_t *rec, float scale, int c, float (&v)[16]) {
+    if (scale < 0.0f) {
+        const f32x4 *const p = reinterpret_cast<const f32x4 *>(rec + 64 * c);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const f32x4 x = p[i];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[4 * i + j] = x[j];
+        }
+        return;
+    }
+    int g, kk[2];
+    kq_place<T>(c, g, kk[0], kk[1]);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const uint8_t *const p = rec + 512 * (kk[h] >> 2) + 16 * (4 * (kk[h] & 3) + g);
+        const f16x8 hi = *reinterpret_cast<const f16x8 *>(p), lo = *reinterpret_cast<const f16x8 *>(p + 256);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {  // slot e holds column 0, 2, 1, 3, 4, 6, 5, 7
+            const int col = (e & 4) | ((e & 1) << 1) | ((e >> 1) & 1);
+            v[8 * h + col] = ((float)hi[e] + (float)lo[e]) * scale;
+        }
+    }
+}
+
 // One item's tile: MT row tiles (cnt routes) x 32 NW weight rows.
 template <int T, int MT, int NW, bool GATED>
 __device__ __forceinline__ void moe_item(const uint8_t *const (&wp)[2], int nsb, const uint8_t *__restrict__ rec,
                                          const uint8_t *__restrict__ mins, const float *__restrict__ scales,
-                                         const int *rows, const int *routes, int cnt, uint8_t *lds, float *out,
-                                         int out_stride, int col) {
+                                         const int *rows, const int *routes, int cnt, uint8_t *lds,
+                                         uint32_t *wide_rows, float *out, int out_stride, int col) {
     using U = KqUnit<2>;
     constexpr int kThreads = 64 * NW;
     constexpr int kBatch = 4, kLoads = 1024 * MT / kThreads, kBatches = (kLoads + kBatch - 1) / kBatch;
@@ -140,6 +182,7 @@ __device__ __forceinline__ void moe_item(const uint8_t *const (&wp)[2], int nsb,
     // A load takes one row's record of the stage per wave (64 pieces).
     v4u st[kBatch], tail;
     float sc = 0.0f;
+    bool wide = false;  // row tid has a wide superblock
     auto load = [&](int bt, int sb) {
 #pragma unroll
         for (int j = 0; j < kBatch; j++) {
@@ -167,10 +210,11 @@ __device__ __forceinline__ void moe_item(const uint8_t *const (&wp)[2], int nsb,
         if constexpr (KqOperand<T, true>::kMins)
             if (tid < 64 * MT)
                 *reinterpret_cast<v4u *>(lds + (b * MT + (tid >> 6)) * U::kBytes + U::kMins + 16 * (tid & 63)) = tail;
+        wide |= sc < 0.0f;
         if (tid < 16 * MT)
             *reinterpret_cast<float *>(lds + (b * MT + (tid >> 4)) * U::kBytes + U::kScales + 4 * (tid & 15)) = sc;
     };
-    kq_stages<T, MT, 2, true>(acc, wp, lds, MT * U::kBytes, 0, nsb, nsb, lane, [](int st) { return st; },
+    kq_stages<T, MT, 2, true, true>(acc, wp, lds, MT * U::kBytes, 0, nsb, nsb, lane, [](int st) { return st; },
                         [&] {  // (requesting W before x is in LDS changed nothing here)
                             load_tail(0);
 #pragma unroll
@@ -191,7 +235,17 @@ __device__ __forceinline__ void moe_item(const uint8_t *const (&wp)[2], int nsb,
                                 store(kBatches - 1, b);
                                 store_tail(b);
                             }
+                        },
+                        [&] {  // (rows past cnt repeat the last route's)
+                            const uint32_t found = (uint32_t)__builtin_amdgcn_ballot_w64(wide && tid < cnt);
+                            if (tid == 0) *wide_rows = found;
                         });
+    if (__builtin_amdgcn_readfirstlane((int)*wide_rows) != 0)
+        kq_wide_rows<T, MT>(wide_rows, acc, wp, 0, nsb, nsb, lane, [](int st) { return st; },
+                            [&](int row, int sb, int c, float (&v)[16]) {
+                                const int64_t rs = (int64_t)rows[row] * nsb + sb;
+                                record_columns<T>(rec + rs * 1024, scales[rs], c, v);
+                            });
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
@@ -227,6 +281,7 @@ __global__ __launch_bounds__(64 * NW) void moe_gemm_kernel(const uint8_t *__rest
     constexpr int kCols = (GATED ? 16 : 32) * NW;
     __shared__ __attribute__((aligned(16))) uint8_t lds[2 * MTMAX * KqUnit<2>::kBytes];
     __shared__ int rows[16 * MTMAX], routes[16 * MTMAX];
+    __shared__ uint32_t wide_rows;  // one bit a row
     const int slices = rows_e / kCols, item = (int)blockIdx.x / slices, slice = (int)blockIdx.x - item * slices;
     if (item >= *nitems) return;
     const int2 it = items[item];
@@ -248,11 +303,11 @@ __global__ __launch_bounds__(64 * NW) void moe_gemm_kernel(const uint8_t *__rest
     const int out_stride = rows_e;
     if constexpr (MTMAX == 2) {
         if (cnt > 16) {
-            moe_item<T, 2, NW, GATED>(wp, nsb, rec, mins, scales, rows, routes, cnt, lds, out, out_stride, col);
+            moe_item<T, 2, NW, GATED>(wp, nsb, rec, mins, scales, rows, routes, cnt, lds, &wide_rows, out, out_stride, col);
             return;
         }
     }
-    moe_item<T, 1, NW, GATED>(wp, nsb, rec, mins, scales, rows, routes, cnt, lds, out, out_stride, col);
+    moe_item<T, 1, NW, GATED>(wp, nsb, rec, mins, scales, rows, routes, cnt, lds, &wide_rows, out, out_stride, col);
 }
 
 namespace {

@@ -303,6 +303,65 @@ def test_gemm_k_quant_tiles(tid, rows, cols, m):
         assert err <= 8e-6
 
 
+def mute_column(tid, data, cols, col):
+    """Codes of column `col` that make its weight 0 in every row (Q6_K: q = 32;
+    Q4_K / Q5_K: scale and min code 0 of its sub-block, one of 0 .. 3)."""
+    b = data.reshape(data.shape[0], cols // 256, -1)
+    sb, e = divmod(col, 256)
+    if tid == syn.Q6_K:
+        h, j, l = e >> 7, (e >> 5) & 3, e & 31
+        ql, qh = 64 * h + 32 * (j & 1) + l, 128 + 32 * h + l
+        b[:, sb, ql] &= 0xF0 if j < 2 else 0x0F
+        b[:, sb, qh] = (b[:, sb, qh] & (255 - (3 << (2 * j)))) | (2 << (2 * j))
+    else:
+        assert e < 128
+        b[:, sb, 4 + e // 32] &= 0xC0
+        b[:, sb, 8 + e // 32] &= 0xC0
+    return data
+
+
+# Activations of a wide range: one element 2^10 .. 2^100 times the rest of its
+# superblock, whose weights are 0, so that the result is what the rest gives;
+# rows of it in the first, a middle and the last row tile, others ordinary, one
+# with a NaN (all of its results NaN), two with an infinity (+-inf and NaN as in
+# the dequantized product).  The rest is held to 2^-19 of the largest of 16
+# columns (1.5e-7 of the result measured) or recomputed in fp32 (K / 64 sums of
+# 64 terms, no more roundings than in test_gemm_k_quant_tiles), so that test's
+# bound holds for each row.
+@pytest.mark.parametrize("tid", [syn.Q4_K, syn.Q5_K, syn.Q6_K])
+@pytest.mark.parametrize("rows,cols,m", [(33, 256, 9), (64, 4608, 16), (50, 768, 17), (1040, 2048, 31), (130, 512, 129),
+                                         (4100, 1024, 333)])
+def test_gemm_k_quant_wide_range(tid, rows, cols, m):
+    import torch
+    print(f"[gpu] k-quant wide range type={tid} rows={rows} cols={cols} m={m}", flush=True)
+    col = cols - 256 + 40
+    data = mute_column(tid, MATRIX[tid](rows, cols, seed=rows + m), cols, col)
+    x = syn.activation_bf16(m, cols, seed=rows + m + 1)
+    wide = dict(zip([0, 1, m // 2, m // 2 + 1, m - 1], [10, 20, 30, 60, 100]))
+    for r, e in wide.items():
+        x[r, col] = (127 + e) << 7  # bf16 2^e
+    x[2, cols - 1] = 0x7F80
+    x[3, col] = 0xFF80
+    x[5, cols - 2] = 0x7FC0
+    with np.errstate(invalid="ignore"):
+        ref = o.gemm_reference(tid, data, cols, x)
+    buf = torch.from_numpy(np.ascontiguousarray(data.reshape(-1))).cuda()
+    xd = torch.from_numpy(x.view(np.int16)).cuda()
+    yd = torch.zeros((m, rows), device="cuda")
+    w = ops.DeviceWeight(tid, buf.data_ptr(), rows, cols)
+    w.gemm_bf16(xd.data_ptr(), m, yd.data_ptr(), stream=torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    y = yd.cpu().numpy()
+    for r in range(m):
+        if r in (2, 3):
+            np.testing.assert_array_equal(y[r].astype(np.float64), ref[r])
+        elif r == 5:
+            assert np.all(np.isnan(y[r]))
+        else:
+            err = np.linalg.norm(y[r] - ref[r]) / np.linalg.norm(ref[r])
+            assert err <= 8e-6, (r, wide.get(r), err)
+
+
 # Q8_0 / Q4_0 on the tile kernel with K a multiple of 32 only: an odd number of
 # blocks (the last 64-column stage holds one; odd rows start on even bytes that
 # are no dword), one block, every tile height, ragged N, y on a dword address.

@@ -9,6 +9,7 @@ import pytest
 from gollek_amd import synthetic as syn
 from gollek_amd import tensor_ops as ops
 from oracle import oracle as o
+from tests.test_gpu_gemm import mute_column
 from tests.test_oracle import (MOE_CF_E, moe_closed_form_case, moe_closed_form_expected,
                                shared_closed_form_case, shared_closed_form_expected)
 
@@ -221,6 +222,52 @@ def test_moe_grouped_gemm(gt, dt, E, H, I, c):
     err = np.linalg.norm(out.astype(np.float64) - ref) / np.linalg.norm(ref)
     print(f"[gpu] moe gemm err={err:.3e} rel_err={o.rel_err(out, ref):.3e}", flush=True)
     assert err <= 2 * 5.7e-6 and o.rel_err(out, ref) <= MOE_TOL
+    for t in (tg, tu, td):
+        t.close()
+
+
+# The grouped GEMM on values of a wide range: x with an element 2^12 .. 2^60
+# times the rest of its superblock whose gate and up weights are 0, h with
+# one (an up row of large d, times its down weights of 0).  The rest is held to
+# 2^-19 of the largest of 16 columns (1.5e-7 of the result measured), or the row
+# is computed in fp32, so test_moe_grouped_gemm's bound holds for each token.  A NaN or an infinity makes
+# every output of its token not finite and leaves the others alone.
+@pytest.mark.parametrize("gt,dt,E,H,I", [(syn.Q4_K, syn.Q4_K, 4, 2816, 1280), (syn.Q4_K, syn.Q6_K, 16, 768, 512),
+                                         (syn.Q5_K, syn.Q5_K, 4, 512, 256), (syn.Q6_K, syn.Q6_K, 16, 1280, 768),
+                                         (syn.Q6_K, syn.Q4_K, 64, 256, 512)])
+def test_moe_grouped_gemm_wide_range(gt, dt, E, H, I):
+    print(f"[gpu] moe gemm wide range gate={gt} down={dt} E={E} H={H} I={I}", flush=True)
+    gate, up, down, *rest = _experts(E, H, I, seed=E + H, down_type=dt, gate_type=gt)
+    for t in rest:
+        t.close()
+    T, k, xcol, hcol = 100, 4, H - 256 + 40, I - 256 + 70
+    gate, up = mute_column(gt, gate, H, xcol), mute_column(gt, up, H, xcol)
+    down = mute_column(dt, down, I, hcol)
+    ublk = up.reshape(E, I, H // 256, -1)
+    at = 208 if gt == syn.Q6_K else 0
+    for a in ((at,) if gt == syn.Q6_K else (0, 2)):  # d (and dmin) 2^20 times as large
+        d = ublk[:, hcol, :, a:a + 2].copy().view(np.float16).astype(np.float32) * 2.0 ** 20
+        assert np.all(np.abs(d) < 65504.0)
+        ublk[:, hcol, :, a:a + 2] = d.astype(np.float16).view(np.uint8)
+    tg, tu, td = (ops.GgufTensor("w", (c, r.shape[0]), t, r.reshape(-1))
+                  for r, c, t in ((gate, H, gt), (up, H, gt), (down, I, dt)))
+    ids, w = syn.moe_routing(T, E, k, seed=71)
+    x = syn.activation(T * H, seed=72).reshape(T, H)
+    wide = {0: 12, 1: 20, 7: 30, 50: 40, T - 1: 60}
+    for t, e in wide.items():
+        x[t, xcol] = 2.0 ** e
+    x[3, xcol] = np.inf
+    x[4, H - 1] = -np.inf
+    x[5, H - 2] = np.nan
+    out = ops.moe_grouped(tg, tu, td, E, x, ids, w)
+    with np.errstate(invalid="ignore"):
+        ref = o.moe_reference_q4k(gate, up, down, E, x, ids, w, down_type=dt, gate_type=gt)
+    for t in range(T):
+        if t in (3, 4, 5):
+            assert not np.any(np.isfinite(out[t]))
+        else:
+            err = np.linalg.norm(out[t].astype(np.float64) - ref[t]) / np.linalg.norm(ref[t])
+            assert err <= 2 * 5.7e-6, (t, wide.get(t), err)
     for t in (tg, tu, td):
         t.close()
 
