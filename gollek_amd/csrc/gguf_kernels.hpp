@@ -180,6 +180,8 @@ constexpr int kMoeMfmaMaxRoutes = 2048;
 // 256, x 16-byte aligned.
 bool moe_kq_mfma_supported(int gate_type, int down_type, int E, int H, int I, int T, int top_k,
                            const float *x);
+// Whether the down rows of a shape it supports take the expert-major pass.
+bool moe_kq_expert_major_down(int down_type, int E, int H, int I, int T, int top_k);
 hipError_t launch_moe_kq_mfma(int gate_type, int down_type, const uint8_t *gate, const uint8_t *up,
                               const uint8_t *down, int E, int H, int I, const float *x, const int32_t *ids,
                               const float *wts, int T, int top_k, float *out, uint8_t *ws, hipStream_t stream);

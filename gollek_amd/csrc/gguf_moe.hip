@@ -868,15 +868,27 @@ hipError_t launch_moe_generic(int gate_type, int up_type, int down_type, const u
 }
 
 // Whether the grouped GEMM's launches (about 45 us with nothing to read) are
-// the faster way: against the two-launch matrix-core passes from three routes
-// per expert and 56 routes (128 experts x 768, hidden 2048, Q4_K: 2 routes per
-// expert 101 us there, 108 here; 4 routes 147 / 119; 16 routes 396 / 166.
-// 64 x 1024, 3 routes: 102 / 77 us; 8 x 1536, 32 routes in all: 38 / 46 us, 64
-// routes: 50 / 46), against the row kernels, which take other shapes, from one
-// (32 x 1280, hidden 2816, Q4_K: 112 / 58 us).
-static bool moe_gemm_chosen(bool tile_passes, int E, int T, int top_k) {
+// the faster way.  Against the row kernels, which take the shapes that the
+// two-launch matrix-core passes do not, from one route per expert (32 x 1280,
+// hidden 2816, Q4_K: 112 / 58 us), if the tokens are enough to share experts:
+// one token's routes, or two tokens' over different experts, are one route each,
+// which the row kernels read as fast without the launches (one Q6_K expert of
+// 5632, hidden 2048: one token 64 / 103 us, two 107 / 106).  Against the
+// two-launch passes from three routes per expert and 56 routes (128 experts x
+// 768, hidden 2048, Q4_K: 4 routes 147 / 119 us, 16 routes 396 / 145; 64 x 1024,
+// 3 routes: 102 / 77 us; 8 x 1536, 32 routes in all: 38 / 46 us, 64 routes: 50 /
+// 46).  Their expert-major down pass holds longer: few experts give the grouped
+// GEMM few workgroups (one of 1536, hidden 2048: Q4_K, 64 routes 46 / 56 us, 80
+// equal; Q5_K, 96 equal; eight experts 56 routes 39 / 41), and with Q5_K down rows it is the faster one up to five
+// routes per expert (128 x 1536, hidden 2048: three 1.34 times as fast, four 1.16,
+// five 0.95; with hidden 1024, x 512, the grouped GEMM from three: 0.78).
+static bool moe_gemm_chosen(bool tile_passes, int down_type, int E, int H, int I, int T, int top_k) {
     const int64_t P = (int64_t)T * top_k;
-    return tile_passes ? P >= 3 * (int64_t)E && P >= 56 : P >= E;
+    if (!tile_passes) return P >= E && (T > 2 || P >= 2 * (int64_t)E);
+    const bool expert_major = moe_kq_expert_major_down(down_type, E, H, I, T, top_k), q5 = down_type == kQ5_K;
+    const int64_t per_expert = expert_major && q5 && H >= 2048 ? 5 : 3;
+    const int64_t least = !expert_major ? 56 : E > 4 ? 64 : q5 ? 96 : 80;
+    return P >= per_expert * E && P >= least;
 }
 
 hipError_t launch_moe(int gate_type, int up_type, int down_type, const uint8_t *gate, const uint8_t *up,
@@ -910,7 +922,7 @@ hipError_t launch_moe(int gate_type, int up_type, int down_type, const uint8_t *
     // take.
     const bool tile_passes = aligned && gate_type == up_type && tuning().moe_variant != 1 &&
                              moe_kq_mfma_supported(gate_type, down_type, E, H, I, T, top_k, x);
-    if (tuning().moe_variant != 1 && moe_gemm_chosen(tile_passes, E, T, top_k) &&
+    if (tuning().moe_variant != 1 && moe_gemm_chosen(tile_passes, down_type, E, H, I, T, top_k) &&
         moe_gemm_supported(gate_type, up_type, down_type, E, H, I, T, top_k, gate, up, down, x))
         return launch_moe_gemm(gate_type, down_type, gate, up, down, E, H, I, x, ids, wts, T, top_k, out, ws, stream);
     if (tile_passes)

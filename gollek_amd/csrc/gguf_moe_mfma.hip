@@ -1793,6 +1793,12 @@ bool moe_kq_mfma_supported(int gate_type, int down_type, int E, int H, int I, in
     return (down_type == kQ4_K || down_type == kQ5_K) && tile_pass_ok(1, E, H, I, down_type);
 }
 
+bool moe_kq_expert_major_down(int down_type, int E, int H, int I, int T, int top_k) {
+    MoeDownGeom gd;
+    int waves = 0;
+    return !token_major_down(down_type, E, H, I, T, top_k, gd, waves);
+}
+
 bool moe_q40_mfma_supported(int E, int H, int I, int P, const float *x) {
     // gate / up rows in one half (hidden up to 2048)
     return H <= 8 * kQK && tile_shape_ok(E, H, I, P, x) && tile_pass_ok(0, E, H, I, kQ4_0) &&

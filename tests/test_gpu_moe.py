@@ -299,6 +299,28 @@ def moe_variant():
     ops.set_option("moe_variant", 0)
 
 
+# One token's routes are one route an expert, whatever the experts' number: the
+# grouped GEMM has nothing to share between them, so shapes that the two-launch
+# passes do not take stay on the row kernels (the same bits as with those forced),
+# as the shared expert of one token does; so do two tokens whose routes may all
+# be of different experts.
+@pytest.mark.parametrize("gt,dt,E,H,I,T,k", [(syn.Q6_K, syn.Q6_K, 2, 2816, 512, 1, 2), (syn.Q4_K, syn.Q6_K, 1, 512, 1280, 1, 1),
+                                             (syn.Q5_K, syn.Q6_K, 4, 4096, 1280, 1, 4), (syn.Q5_K, syn.Q6_K, 4, 512, 1280, 2, 2)])
+def test_moe_single_routes_take_the_row_kernels(gt, dt, E, H, I, T, k, moe_variant):
+    print(f"[gpu] moe single routes gate={gt} down={dt} E={E} H={H} I={I} T={T}", flush=True)
+    *_, tg, tu, td = _experts(E, H, I, seed=E + H, down_type=dt, gate_type=gt)
+    ids, w = syn.moe_routing(T, E, k, seed=81)
+    x = syn.activation(T * H, seed=82).reshape(T, H)
+    out = ops.moe_grouped(tg, tu, td, E, x, ids, w)
+    shared = ops.moe_shared_expert(tg, tu, td, x, np.zeros_like(x)) if E == 1 else None
+    moe_variant(1)
+    np.testing.assert_array_equal(out, ops.moe_grouped(tg, tu, td, E, x, ids, w))
+    if E == 1:
+        np.testing.assert_array_equal(shared, ops.moe_shared_expert(tg, tu, td, x, np.zeros_like(x)))
+    for t in (tg, tu, td):
+        t.close()
+
+
 @pytest.mark.parametrize("gt,dt", [(syn.Q4_0, syn.Q4_0), (syn.Q5_K, syn.Q6_K), (syn.Q5_K, syn.Q5_K),
                                    (syn.Q6_K, syn.Q6_K)])
 def test_moe_matrix_core_equals_row_kernels(gt, dt, moe_variant):
