@@ -399,7 +399,9 @@ bool moe_gemm_supported(int gate_type, int up_type, int down_type, int E, int H,
     const int64_t items = max_items(P, E, 16 * item_tiles(P, E));
     const RecordTails xt = tails_at(L.xdig, T, H / kQK);
     return (xt.end + 15) / 16 * 16 + (size_t)items * 8 <= L.h && tails_at(L.hdig, P, I / kQK).end <= L.ypair &&
-           items * (H / 64) < ((int64_t)1 << 31) && (P + 15) / 16 <= 65535;
+           (P + 15) / 16 <= 65535 &&
+           // threads of the passes: four a gate row and item, two a down row
+           items * (4 * (int64_t)I > 2 * (int64_t)H ? 4 * (int64_t)I : 2 * (int64_t)H) < ((int64_t)1 << 32);
 }
 
 hipError_t launch_moe_gemm(int gate_type, int down_type, const uint8_t *gate, const uint8_t *up, const uint8_t *down,
