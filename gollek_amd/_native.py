@@ -78,11 +78,12 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "gollek_hip_gguf_upload": (_P, [_P, _I64, _CHARP, _SZ]),
 }
 
-# Test-only export (gollek_amd/csrc/gollek_hip_testing.h; not part of the
-# drop-in ABI): forces a GEMV / MoE kernel family onto shapes another one
-# is picked for, so the parity tests reach every family.
+# Test-only exports (gollek_amd/csrc/gollek_hip_testing.h; not part of the
+# drop-in ABI): one forces a GEMV / MoE kernel family onto shapes another one
+# is picked for, so the parity tests reach every family; one tells a GEMM's tiles.
 TESTING_SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "gollek_hip_testing_set_option": (_I32, [_CHARP, _I64, _CHARP, _SZ]),
+    "gollek_hip_testing_gemm_plan": (_I32, [_I32, _I64, _I64, _I64, _P]),
 }
 
 _lock = threading.Lock()

@@ -322,6 +322,18 @@ int32_t gollek_hip_testing_set_option(const char *key, int64_t value, char *err,
     return GOLLEK_HIP_OK;
 }
 
+int32_t gollek_hip_testing_gemm_plan(int32_t type_id, int64_t m, int64_t n, int64_t k, int32_t *plan) {
+    if (plan == nullptr || m < 1 || n < 1 || k < 1 || m > INT32_MAX || n > INT32_MAX || k > INT32_MAX)
+        return GOLLEK_HIP_ERR_ARG;
+    int32_t p[4];
+    if (type_id == GOLLEK_HIP_Q8_0 || type_id == GOLLEK_HIP_Q4_0)
+        gollek::gemm_tile_plan(type_id, (int)m, (int)n, (int)k, p);
+    else if (supported(type_id)) gollek::kq_gemm_plan(type_id, (int)m, (int)n, (int)k, p);
+    else return GOLLEK_HIP_ERR_UNSUPPORTED;
+    for (int i = 0; i < 4; i++) plan[i] = p[i];
+    return GOLLEK_HIP_OK;
+}
+
 gollek_hip_weight *gollek_hip_weight_upload(int32_t type_id, const void *host_bytes, int64_t rows,
                                             int64_t cols, int64_t row_bytes, char *err,
                                             size_t err_len) {

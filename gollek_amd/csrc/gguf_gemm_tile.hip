@@ -567,6 +567,12 @@ size_t gemm_tile_workspace_bytes(int type_id, int M, int N, int K) {
     return S > 1 ? (size_t)(S - 1) * M * N * sizeof(float) : 0;
 }
 
+void gemm_tile_plan(int type_id, int M, int N, int K, int32_t (&plan)[4]) {
+    plan[0] = tile_mt(type_id, M, N, K);
+    plan[1] = plan[2] = 0;
+    plan[3] = ((int64_t)M * N) % 4 == 0 ? tile_splits(type_id, M, N, K, (size_t)-1) : 1;
+}
+
 hipError_t launch_gemm_tile(int type_id, const uint8_t *w, int64_t row_bytes, const uint16_t *x,
                             float *y, int M, int N, int K, hipStream_t stream, float *workspace,
                             size_t workspace_bytes) {

@@ -125,12 +125,16 @@ bool gemm_may_split(int type_id, int M, int N, int K);
 // multiple of 256, x 16-byte and W rows 2-byte aligned.
 bool kq_gemm_supported(int type_id, int64_t row_bytes, int N, int K, const void *w, const void *x);
 size_t kq_gemm_workspace_bytes(int type_id, int M, int N, int K);
+// The plan of a call whose buffers are aligned and whose workspace suffices, for
+// the tests: {row tiles, column waves, K waves, K splits}.
+void kq_gemm_plan(int type_id, int M, int N, int K, int32_t (&plan)[4]);
 hipError_t launch_kq_gemm(int type_id, const uint8_t *w, int64_t row_bytes, const uint16_t *x, float *y, int M, int N,
                           int K, hipStream_t stream, float *workspace, size_t workspace_bytes);
 // The 128 x 128 tile kernel of Q8_0 and Q4_0 (gguf_gemm_tile.hip): K a
 // multiple of 32, W 4-byte aligned with rows on even bytes, x 16-byte aligned.
 bool gemm_tile_supported(int type_id, int64_t row_bytes, int M, int N, int K, const void *w, const void *x);
 size_t gemm_tile_workspace_bytes(int type_id, int M, int N, int K);
+void gemm_tile_plan(int type_id, int M, int N, int K, int32_t (&plan)[4]);  // {row tiles, 0, 0, K splits}
 hipError_t launch_gemm_tile(int type_id, const uint8_t *w, int64_t row_bytes, const uint16_t *x,
                             float *y, int M, int N, int K, hipStream_t stream, float *workspace,
                             size_t workspace_bytes);

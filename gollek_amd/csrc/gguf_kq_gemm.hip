@@ -288,6 +288,15 @@ size_t kq_gemm_workspace_bytes(int type_id, int M, int N, int K) {
     return gemm_plan_bytes(kq_plan(type_id, M, N, K, kGemmMaxSplitBytes), M, N);
 }
 
+void kq_gemm_plan(int type_id, int M, int N, int K, int32_t (&plan)[4]) {
+    const bool split = gemm_may_split(type_id, M, N, K) && ((int64_t)M * N) % 4 == 0;
+    const GemmPlan p = kq_plan(type_id, M, N, K, split ? kGemmMaxSplitBytes : 0);
+    plan[0] = p.mt;
+    plan[1] = p.nw;
+    plan[2] = p.kw;
+    plan[3] = p.splits;
+}
+
 hipError_t launch_kq_gemm(int type_id, const uint8_t *w, int64_t row_bytes, const uint16_t *x, float *y, int M, int N,
                           int K, hipStream_t stream, float *workspace, size_t workspace_bytes) {
     const bool split = workspace != nullptr && gemm_may_split(type_id, M, N, K) && ((int64_t)M * N) % 4 == 0 &&

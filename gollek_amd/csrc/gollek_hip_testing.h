@@ -1,5 +1,5 @@
 /*
- * gollek_hip_testing.h -- test-only export of libgollek_hip.so; not part of
+ * gollek_hip_testing.h -- test-only exports of libgollek_hip.so; not part of
  * the drop-in C ABI (include/gollek_hip.h), and the Java adapter never binds
  * it.
  *
@@ -28,6 +28,13 @@ extern "C" {
 #endif
 
 int32_t gollek_hip_testing_set_option(const char *key, int64_t value, char *err, size_t err_len);
+
+/* The tiles that a GEMM of m x n outputs and k columns takes on its type's tile
+ * kernel (aligned buffers, the full workspace; no device is needed, 256 compute
+ * units until one is initialised), so that the tests can tell which kernels
+ * their shapes reach: plan[4] = {row tiles of 16, column waves, K waves, K
+ * splits} for the K-quants, {row tiles of 16, 0, 0, K splits} for Q8_0 / Q4_0. */
+int32_t gollek_hip_testing_gemm_plan(int32_t type_id, int64_t m, int64_t n, int64_t k, int32_t *plan);
 
 #ifdef __cplusplus
 }

@@ -1,5 +1,5 @@
-"""GPU parity of the Q8_0 / Q4_0 / Q4_K / Q5_K x bf16 MFMA GEMM and the Q6_K
-fp32 MFMA GEMM (small-M prefill / batched decode).
+"""GPU parity of the GEMM (small-M prefill / batched decode): Q8_0 / Q4_0 on
+the bf16 matrix cores, the K-quants on the fp16 ones, other alignments in fp32.
 
 Bar: rel_err <= 1e-2 against the fp64 product of the bf16 activations and the
 bit-exact dequantized weights (the quants are contracted exactly and each
@@ -120,12 +120,13 @@ def _gemm_case(type_id, rows, cols, m, seed):
 @pytest.mark.parametrize("rows,cols,m", [(128, 256, 33), (192, 4096, 300), (80, 512, 129), (4096, 256, 257),
                                           (1000, 1024, 64), (256, 2048, 1024), (64, 4096, 40), (300, 1024, 96)])
 def test_gemm_tile_kernel_shapes(type_id, rows, cols, m):
-    # The tile kernel (16 MT x 128 tiles: MT = 8 past M = 64, 4 for M = 33
-    # .. 64 and for Q8_0 up to 128 when N has at most 32 column tiles, as
-    # at M = 96 here): K from one four-stage round (256) up, a
+    # The tile kernels.  Q8_0 / Q4_0 (16 MT x 128 tiles: MT = 8 past M = 64, 4
+    # for M = 33 .. 64 and for Q8_0 up to 128 when N has at most 32 column
+    # tiles, as at M = 96 here): K from one four-stage round (256) up, a
     # partial last M tile (rows past M read zeros) and N tile (rows past N),
     # one to many tiles, grids that are and are not a multiple of 8, and the
-    # K splits the CU count allows (none for K = 256, up to 8).
+    # K splits the CU count allows (none for K = 256, up to 8).  The K-quants
+    # take the plans of gguf_gemm_plan.hpp (test_gemm_k_quant_tiles).
     print(f"[gpu] gemm tile type={type_id} rows={rows} cols={cols} m={m}", flush=True)
     y, ref = _gemm_case(type_id, rows, cols, m, seed=rows + 3 * cols + m + type_id)
     err = o.rel_err(y, ref)
@@ -137,8 +138,9 @@ def test_gemm_tile_kernel_shapes(type_id, rows, cols, m):
 @pytest.mark.parametrize("rows,cols,m", [(100, 512, 5), (1000, 1024, 16), (64, 256, 1), (200, 2048, 32),
                                           (520, 4096, 17), (3000, 4096, 48), (14336, 4096, 8)])
 def test_gemm_tile_kernel_small_m(type_id, rows, cols, m):
-    # Tiles of 16, 32 and 64 rows of X for M up to 16, 32 and 64 (Q8_0 with
-    # 16-row multiples of N and M <= 32 takes the skinny kernel instead).
+    # Q8_0 / Q4_0: tiles of 16, 32 and 64 rows of X for M up to 16, 32 and 64
+    # (Q8_0 with 16-row multiples of N and M <= 32 takes the skinny kernel
+    # instead).  K-quants: the plans of small M.
     print(f"[gpu] gemm small-m type={type_id} rows={rows} cols={cols} m={m}", flush=True)
     y, ref = _gemm_case(type_id, rows, cols, m, seed=rows + 5 * cols + m + type_id)
     err = o.rel_err(y, ref)
@@ -164,9 +166,9 @@ def test_gemm_q4_parity_14336(type_id, m):
     [(syn.Q4_0, 48, 96, 3), (syn.Q4_0, 16, 64, 20), (syn.Q4_0, 40, 512, 7), (syn.Q4_0, 20, 768, 5),
      (syn.Q4_K, 40, 512, 7), (syn.Q4_K, 20, 768, 5)])
 def test_gemm_q4_generic_shapes(type_id, rows, cols, m):
-    # K = 64 and 96 are not multiples of 256: the one-thread-per-output
-    # kernel.  K = 512 and 768 with fewer than 128 rows and tokens: one
-    # partial tile of the tile kernel.
+    # K = 64 and 96: whole and half 64-column stages of the tile kernel, unsplit
+    # (the one-thread-per-output kernels take unaligned X, below).  K = 512 and
+    # 768 with fewer than 128 rows and tokens: one partial tile.
     print(f"[gpu] gemm generic type={type_id} rows={rows} cols={cols} m={m}", flush=True)
     y, ref = _gemm_case(type_id, rows, cols, m, seed=rows + cols + m)
     assert o.rel_err(y, ref) <= GEMM_TOL
@@ -175,7 +177,7 @@ def test_gemm_q4_generic_shapes(type_id, rows, cols, m):
 def test_gemm_q4k_special_headers():
     # Q4_K superblocks with zero min codes under a NaN dmin (the min term is
     # skipped, as RT/GgufKQuantLayout.java:67-69), zero d, and a subnormal
-    # dmin: the tile kernel equals the fp64 product of the bit-exact rows.
+    # dmin: the K-quant kernel equals the fp64 product of the bit-exact rows.
     rows, cols, m = 256, 1024, 160
     data = syn.q4_k_matrix(rows, cols, seed=17).copy()
     blocks = data.reshape(rows, cols // 256, 144)
@@ -225,10 +227,10 @@ def test_gemm_split_k_shapes(rows, cols, m):
     t.close()
 
 
-# Q6_K weights (the Q6_K tensors of Q4_K_M files): the tile kernel for rows
-# of an even superblock count (superblocks of odd index start 2 bytes past a
-# dword; K = 14336 and M = 512 too), the fp32 matrix-core kernel for odd
-# counts (K = 768), with partial tiles on both sides.
+# Q6_K weights (the Q6_K tensors of Q4_K_M files): rows of an even superblock
+# count (superblocks of odd index start 2 bytes past a dword; K = 14336 and M =
+# 512 too) and of an odd one (K = 768: every other row does), with partial tiles
+# on both sides.
 @pytest.mark.parametrize("tid,rows,cols,m", [(syn.Q6_K, 4096, 4096, 16), (syn.Q6_K, 33, 768, 1),
                                              (syn.Q6_K, 1024, 4096, 128), (syn.Q6_K, 100, 512, 37),
                                              (syn.Q6_K, 4096, 14336, 24), (syn.Q6_K, 14336, 4096, 512)])
@@ -247,8 +249,8 @@ def test_gemm_q5_k_q6_k(tid, rows, cols, m):
 
 @pytest.mark.parametrize("tid", [syn.Q5_K, syn.Q6_K])
 def test_gemm_k_quant_unaligned_x_takes_the_generic_kernel(tid):
-    # x 2 bytes past a 16-byte boundary: the Q5_K tile kernel's loads need
-    # 16 and the Q6_K kernel's 4, so the device entry runs the per-output
+    # x 2 bytes past a 16-byte boundary: the K-quant kernel's loads need 16 and
+    # the fp32 Q6_K kernel's 4, so the device entry runs the per-output
     # fp32 kernel (gemm_kquant_generic_kernel), with the same values.
     import torch
     rows, cols, m = 272, 1024, 9
@@ -267,17 +269,49 @@ def test_gemm_k_quant_unaligned_x_takes_the_generic_kernel(tid):
         dw.close()
 
 
-# The K-quant kernel at the edges of its tiles: row tiles of 16 (M around
-# them, 96 = 6 and 128 = 8 of them), ragged column groups of 32, superblock
-# counts that its waves' slices do not divide, K split over workgroups
-# (N = 64, 1040), weights on even but not dword addresses and y on dword but
-# not 16-byte ones (runs unsplit).  Norm-wise bound: every product is exact, a
-# sum takes 256 additions in the matrix core and K / 256 (at most 17) outside of
-# 2^-24 each, random in sign, with terms up to 8 times the result
-# (d P against dmin PM): 8 * sqrt(273) * 2^-24 = 8e-6.
+# X that is not 16-byte aligned.  2 bytes off: one thread per output
+# (gemm_q8_0_generic_kernel, gemm_generic_kernel, gemm_kquant_generic_kernel); 4
+# bytes off: the same, and Q6_K on the fp32 matrix cores (gemm_q6k_f32_kernel: X
+# tiles of 16, 32 and 64 rows, and 64 x 64 tiles where those give every CU two
+# workgroups, N = 2112 at M = 1000).
+@pytest.mark.parametrize("off", [1, 2])
+@pytest.mark.parametrize("tid,rows,cols,m", [
+    (syn.Q8_0, 272, 1024, 9), (syn.Q8_0, 50, 96, 40), (syn.Q4_0, 272, 1024, 9), (syn.Q4_0, 50, 64, 33),
+    (syn.Q4_K, 272, 1024, 9), (syn.Q5_K, 272, 1024, 9), (syn.Q6_K, 272, 1024, 9), (syn.Q6_K, 33, 768, 20),
+    (syn.Q6_K, 100, 512, 40), (syn.Q6_K, 2112, 256, 1000)])
+def test_gemm_unaligned_x(tid, rows, cols, m, off):
+    import torch
+    print(f"[gpu] gemm unaligned x type={tid} rows={rows} cols={cols} m={m} off={2 * off}", flush=True)
+    data = syn.matrix(tid, rows, cols, 77)
+    x = syn.activation_bf16(m, cols, seed=78)
+    w_dev = torch.from_numpy(data.reshape(-1)).cuda()
+    dw = ops.DeviceWeight(tid, w_dev.data_ptr(), rows, cols)
+    try:
+        buf = torch.zeros(m * cols + 8, dtype=torch.int16, device="cuda")
+        buf[off:off + m * cols] = torch.from_numpy(x.view(np.int16).reshape(-1)).cuda()
+        y_dev = torch.full((m, rows), float("nan"), dtype=torch.float32, device="cuda")
+        dw.gemm_bf16(buf.data_ptr() + 2 * off, m, y_dev.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert o.rel_err(y_dev.cpu().numpy(), o.gemm_reference(tid, data, cols, x)) <= GEMM_TOL
+    finally:
+        dw.close()
+
+
+# The K-quant kernel at the edges of its tiles: M around row tiles of 16, ragged
+# column groups of 32, superblock counts that its waves' slices do not divide,
+# every plan (test_gemm_plans.py tells which shape reaches which), K split over
+# workgroups (64 x 4608, 2080 x 4608), weights on even but not dword addresses
+# and y on dword but not 16-byte ones (runs unsplit).  Norm-wise bound: every
+# product is exact, a sum takes 256 additions in the matrix core and K / 256
+# outside of 2^-24 each, random in sign, with terms up to 8 times the result
+# (d P against dmin PM): 8 * sqrt(256 + K / 256) * 2^-24, 8e-6 at K = 4352.
+K_QUANT_TILES = [(33, 256, 5), (64, 4352, 16), (50, 768, 17), (300, 1280, 33), (1040, 2048, 31), (2080, 768, 96),
+                 (130, 512, 129), (4100, 1024, 333), (64, 4608, 16), (33, 8192, 5), (300, 512, 600), (300, 2048, 1000),
+                 (1040, 768, 700), (4100, 768, 600), (2080, 4608, 600), (14336, 768, 500)]
+
+
 @pytest.mark.parametrize("tid", [syn.Q4_K, syn.Q5_K, syn.Q6_K])
-@pytest.mark.parametrize("rows,cols,m", [(33, 256, 5), (64, 4352, 16), (50, 768, 17), (300, 1280, 33), (1040, 2048, 31),
-                                         (2080, 768, 96), (130, 512, 129), (4100, 1024, 333)])
+@pytest.mark.parametrize("rows,cols,m", K_QUANT_TILES)
 def test_gemm_k_quant_tiles(tid, rows, cols, m):
     import torch
     print(f"[gpu] k-quant gemm type={tid} rows={rows} cols={cols} m={m}", flush=True)
@@ -300,7 +334,7 @@ def test_gemm_k_quant_tiles(tid, rows, cols, m):
         assert np.all(y[:y_off] == 0.0) and np.all(y[y_off + m * rows:] == 0.0)
         err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
         print(f"[gpu] k-quant gemm err={err:.2e}", flush=True)
-        assert err <= 8e-6
+        assert err <= 8 * np.sqrt(256 + cols // 256) * 2.0 ** -24
 
 
 def mute_column(tid, data, cols, col):
@@ -364,13 +398,17 @@ def test_gemm_k_quant_wide_range(tid, rows, cols, m):
 
 # Q8_0 / Q4_0 on the tile kernel with K a multiple of 32 only: an odd number of
 # blocks (the last 64-column stage holds one; odd rows start on even bytes that
-# are no dword), one block, every tile height, ragged N, y on a dword address.
+# are no dword), one block, every tile height (test_gemm_plans.py), ragged N, y
+# on a dword address.
 # Norm-wise bound: exact products, K / 32 (at most 91) roundings of 2^-24, random
 # in sign, of terms no larger than the result's norm: 10 * 2^-24 and twice
 # that for the matrix core's own sums.
+RAGGED_K = [(33, 32, 1), (130, 96, 17), (300, 2912, 5), (129, 1056, 64), (1000, 864, 65), (4000, 2912, 130),
+            (5760, 2880, 100), (70, 64, 600), (2001, 864, 600), (4100, 1056, 700)]
+
+
 @pytest.mark.parametrize("tid", [syn.Q8_0, syn.Q4_0])
-@pytest.mark.parametrize("rows,cols,m", [(33, 32, 1), (130, 96, 17), (300, 2912, 5), (129, 1056, 64), (1000, 864, 65),
-                                         (4000, 2912, 130), (5760, 2880, 100), (70, 64, 600)])
+@pytest.mark.parametrize("rows,cols,m", RAGGED_K)
 def test_gemm_ragged_k(tid, rows, cols, m):
     import torch
     print(f"[gpu] ragged gemm type={tid} rows={rows} cols={cols} m={m}", flush=True)
@@ -445,12 +483,15 @@ def test_gemm_device_entry_split_k_workspace(m):
         dw.close()
 
 
-@pytest.mark.parametrize("type_id,rows,m", [(syn.Q8_0, 4096, 512), (syn.Q4_K, 4096, 512), (syn.Q4_0, 2048, 1024),
-                                           (syn.Q5_K, 4096, 128), (syn.Q6_K, 4096, 128)])
+SPLIT_REPEATS = [(syn.Q8_0, 4096, 512), (syn.Q4_K, 4096, 128), (syn.Q4_0, 2048, 1024), (syn.Q5_K, 4096, 128),
+                 (syn.Q6_K, 4096, 128)]
+
+
+@pytest.mark.parametrize("type_id,rows,m", SPLIT_REPEATS + [(syn.Q4_K, 4096, 512)])
 def test_gemm_two_split_repeatable(type_id, rows, m):
-    # Two K splits added in split order by the reduction kernel: the same
-    # bits on every call, within the bar of the oracle, on repeated calls
-    # with the handle's workspace reused.
+    # K splits (two; Q5_K, Q6_K four; Q4_K at M = 512 none) added in split order
+    # by the reduction kernel: the same bits on every call, within the bar of
+    # the oracle, on repeated calls with the handle's workspace reused.
     import torch
     cols = 4096
     data = MATRIX[type_id](rows, cols, seed=rows + m)

@@ -168,11 +168,12 @@ def test_moe_q6_k_gate_up_parity(dt, E, H, I, T, k):
         t.close()
 
 
-# Prefill: more than 2048 routes (tokens x top_k) run the matrix-core passes
-# over token slices of 2048 / top_k tokens (256 + 44 at top-8, 512 + 88 at
-# top-4, 1024 + 76 and 1024 + 6 at top-2; expert-major down at inter 1280).
-# A token's output depends on its own routes only, so the sliced call equals,
-# bit for bit, one call per slice, and both are within the bar of the oracle.
+# Prefill: more than 2048 routes (tokens x top_k) run as token slices of 2048 /
+# top_k tokens (256 + 44 at top-8, 512 + 88 at top-4, 1024 + 76 and 1024 + 6 at
+# top-2), each K-quant slice on the grouped GEMM or, with few routes (the last
+# 12), the matrix-core passes.  A token's output depends on its own routes only,
+# so the sliced call equals, bit for bit, one call per slice, and both are within
+# the bar of the oracle.
 @pytest.mark.parametrize("gt,dt,E,H,I,T,k", [
     (syn.Q4_K, syn.Q4_K, 32, 512, 256, 300, 8), (syn.Q5_K, syn.Q6_K, 16, 1024, 512, 600, 4),
     (syn.Q4_0, syn.Q4_0, 32, 512, 256, 1100, 2), (syn.Q4_K, syn.Q5_K, 8, 512, 1280, 1030, 2)])
@@ -268,6 +269,26 @@ def test_moe_grouped_gemm_wide_range(gt, dt, E, H, I):
         else:
             err = np.linalg.norm(out[t].astype(np.float64) - ref[t]) / np.linalg.norm(ref[t])
             assert err <= 2 * 5.7e-6, (t, wide.get(t), err)
+    for t in (tg, tu, td):
+        t.close()
+
+
+# The grouped GEMM's routing: runs of routes scattered by 16 waves with the keys
+# in LDS, the same with more keys than fit it (16400 routes), and one wave past
+# 512 experts.  (Q6_K rows of one superblock: a shape of the row kernels, so all
+# routes are one call's.)  The bound of test_moe_grouped_gemm.
+@pytest.mark.parametrize("E,T,k", [(16, 700, 2), (4, 8200, 2), (520, 300, 2)])
+def test_moe_grouped_gemm_routing(E, T, k):
+    print(f"[gpu] moe gemm routing E={E} T={T} k={k}", flush=True)
+    gate, up, down, tg, tu, td = _experts(E, 256, 256, seed=E + T, down_type=syn.Q6_K, gate_type=syn.Q6_K)
+    ids, w = syn.moe_routing(T, E, k, seed=91)
+    ids[T // 2, 0], w[T // 3, 1] = E, 0.0
+    x = syn.activation(T * 256, seed=92).reshape(T, 256)
+    out = ops.moe_grouped(tg, tu, td, E, x, ids, w)
+    ref = o.moe_reference_q4k(gate, up, down, E, x, ids, w, down_type=syn.Q6_K, gate_type=syn.Q6_K)
+    err = np.linalg.norm(out.astype(np.float64) - ref) / np.linalg.norm(ref)
+    print(f"[gpu] moe gemm routing err={err:.3e}", flush=True)
+    assert err <= 2 * 5.7e-6
     for t in (tg, tu, td):
         t.close()
 
@@ -422,12 +443,14 @@ def _nan_dmin_zero_mins(blocks, pb, rows, every=3):
 
 
 # K-quant experts whose superblocks carry a NaN dmin with all min codes 0:
-# the matrix-core passes' non-finite branch (and the row kernels) give the
-# reference's finite values for them, on gate / up and on Q4_K / Q5_K down rows.
+# the matrix-core passes' non-finite branch (and the row kernels, and the grouped
+# GEMM, with 80 routes) give the reference's finite values for them, on gate / up
+# and on Q4_K / Q5_K down rows.
+@pytest.mark.parametrize("T", [5, 40])
 @pytest.mark.parametrize("gt,dt", [(syn.Q4_K, syn.Q4_K), (syn.Q5_K, syn.Q6_K), (syn.Q5_K, syn.Q5_K),
                                    (syn.Q4_K, syn.Q5_K)])
-def test_moe_nan_dmin_with_zero_min_codes(gt, dt):
-    E, H, I, T, k = 8, 512, 256, 5, 2
+def test_moe_nan_dmin_with_zero_min_codes(gt, dt, T):
+    E, H, I, k = 8, 512, 256, 2
     pb = {syn.Q4_K: 144, syn.Q5_K: 176}
     gate = syn.matrix(gt, E * I, H, 61)
     up = syn.matrix(gt, E * I, H, 62)

@@ -5,11 +5,12 @@ partials in the library's static per-GPU scratch instead of the handle's
 workspace, so its output must equal the allocating entry point's bit for
 bit, and both must be within the GEMM bar (rel_err <= 1e-2) of the fp64
 oracle.  Calls in a row on one handle, each with fewer rows of X than the
-one before, all split over K so all use the scratch, and none may read an
+one before, split over K so that they use the scratch, and none may read an
 earlier call's partials: Q8_0 at 4096 rows (m = 512 with two splits, the
-others with more), Q4_K at 14336 rows (m = 128 in 128-row tiles, m = 16 in
-16-row tiles), Q4_0 at 4096 rows (m = 300, then 20 in 32-row tiles) and
-Q5_K at 4096 rows (m = 64, then 16); Q6_K (the fp32 kernel, no split) too.
+others with more), Q4_K at 4096 rows (m = 128 with two splits, 16 with four),
+Q4_0 at 4096 rows (m = 300, then 20 in 32-row tiles), Q5_K at 4096 rows (m =
+64, then 16) and Q6_K at 1024 (m = 37, then 5); Q4_K at 14336 rows, which does
+not split, too.
 """
 import ctypes
 
@@ -26,11 +27,11 @@ pytestmark = pytest.mark.gpu
 GEMM_TOL = 1e-2
 
 
-@pytest.mark.parametrize("type_id,rows,cols,ms", [(syn.Q8_0, 4096, 4096, (512, 200, 48)),
-                                                  (syn.Q4_K, 14336, 4096, (128, 16)),
-                                                  (syn.Q4_0, 4096, 4096, (300, 20)),
-                                                  (syn.Q5_K, 4096, 4096, (64, 16)),
-                                                  (syn.Q6_K, 1024, 2048, (37, 5))])
+SPLIT = [(syn.Q8_0, 4096, 4096, (512, 200, 48)), (syn.Q4_K, 4096, 4096, (128, 16)), (syn.Q4_0, 4096, 4096, (300, 20)),
+         (syn.Q5_K, 4096, 4096, (64, 16)), (syn.Q6_K, 1024, 2048, (37, 5))]
+
+
+@pytest.mark.parametrize("type_id,rows,cols,ms", SPLIT + [(syn.Q4_K, 14336, 4096, (128, 16))])
 def test_noalloc_gemm_matches_allocating_entry_point(type_id, rows, cols, ms):
     import torch
 
