@@ -225,23 +225,23 @@ namespace {
 
 // Fitted per type (gguf_gemm_plan.hpp).
 constexpr GemmPlanCost kQ4KPlans[] = {
-    {1, 1, 4, 2, 3.36f, 2.71f}, {1, 1, 8, 1, 3.73f, 2.95f}, {1, 2, 4, 1, 2.20f, 2.19f},
-    {2, 2, 2, 2, 3.06f, 3.05f}, {2, 2, 4, 1, 3.82f, 3.25f}, {2, 4, 2, 1, 2.55f, 2.47f},
-    {4, 4, 2, 1, 4.02f, 3.73f}, {4, 8, 1, 1, 2.43f, 2.99f}, {6, 8, 1, 1, 3.60f, 3.94f},
-    {8, 8, 1, 1, 4.25f, 4.91f}};
-constexpr GemmSplitCost kQ4KSplit = {1.80f, 0.277f};
+    {1, 1, 4, 2, 3.30f, 2.87f}, {1, 1, 8, 1, 2.70f, 3.17f}, {1, 2, 4, 1, 2.19f, 2.19f},
+    {2, 2, 2, 2, 3.90f, 3.25f}, {2, 2, 4, 1, 2.98f, 3.31f}, {2, 4, 2, 1, 2.94f, 2.51f},
+    {4, 4, 2, 1, 4.18f, 3.71f}, {4, 8, 1, 1, 3.77f, 2.96f}, {6, 8, 1, 1, 5.51f, 3.73f},
+    {8, 8, 1, 1, 6.48f, 5.01f}};
+constexpr GemmSplitCost kQ4KSplit = {2.88f, 0.179f};
 constexpr GemmPlanCost kQ5KPlans[] = {
-    {1, 1, 4, 2, 4.32f, 3.50f}, {1, 1, 8, 1, 4.44f, 3.96f}, {1, 2, 4, 1, 2.97f, 3.03f},
-    {2, 2, 2, 2, 3.96f, 3.81f}, {2, 2, 4, 1, 4.61f, 4.20f}, {2, 4, 2, 1, 3.39f, 3.34f},
-    {4, 4, 2, 1, 4.77f, 4.61f}, {4, 8, 1, 1, 3.64f, 3.79f}, {6, 8, 1, 1, 4.04f, 4.96f},
-    {8, 8, 1, 1, 5.17f, 5.97f}};
-constexpr GemmSplitCost kQ5KSplit = {1.73f, 0.295f};
+    {1, 1, 4, 2, 3.49f, 3.74f}, {1, 1, 8, 1, 2.65f, 4.14f}, {1, 2, 4, 1, 2.23f, 3.24f},
+    {2, 2, 2, 2, 3.55f, 4.06f}, {2, 2, 4, 1, 2.88f, 4.32f}, {2, 4, 2, 1, 3.03f, 3.40f},
+    {4, 4, 2, 1, 3.86f, 4.71f}, {4, 8, 1, 1, 3.64f, 3.69f}, {6, 8, 1, 1, 4.70f, 4.79f},
+    {8, 8, 1, 1, 5.19f, 5.66f}};
+constexpr GemmSplitCost kQ5KSplit = {2.85f, 0.218f};
 constexpr GemmPlanCost kQ6KPlans[] = {
-    {1, 1, 4, 2, 4.59f, 4.39f}, {1, 1, 8, 1, 4.60f, 4.80f}, {1, 2, 4, 1, 3.62f, 4.03f},
-    {2, 2, 2, 2, 4.00f, 4.52f}, {2, 2, 4, 1, 4.51f, 5.15f}, {2, 4, 2, 1, 3.30f, 4.60f},
-    {4, 4, 2, 1, 4.29f, 5.48f}, {4, 8, 1, 1, 3.59f, 5.15f}, {6, 8, 1, 1, 3.89f, 6.27f},
-    {8, 8, 1, 1, 5.83f, 8.54f}};
-constexpr GemmSplitCost kQ6KSplit = {2.43f, 0.297f};
+    {1, 1, 4, 2, 2.90f, 4.64f}, {1, 1, 8, 1, 2.64f, 5.33f}, {1, 2, 4, 1, 2.15f, 4.68f},
+    {2, 2, 2, 2, 3.17f, 4.65f}, {2, 2, 4, 1, 2.92f, 5.39f}, {2, 4, 2, 1, 2.59f, 4.59f},
+    {4, 4, 2, 1, 3.66f, 5.65f}, {4, 8, 1, 1, 3.57f, 5.04f}, {6, 8, 1, 1, 4.62f, 6.15f},
+    {8, 8, 1, 1, 5.23f, 7.90f}};
+constexpr GemmSplitCost kQ6KSplit = {2.97f, 0.203f};
 
 GemmPlan kq_plan(int type_id, int M, int N, int K, size_t ws_bytes) {
     if (type_id == kQ4_K) return pick_gemm_plan(kQ4KPlans, kQ4KSplit, M, N, K, ws_bytes);

@@ -7,10 +7,10 @@ bit, and both must be within the GEMM bar (rel_err <= 1e-2) of the fp64
 oracle.  Calls in a row on one handle, each with fewer rows of X than the
 one before, split over K so that they use the scratch, and none may read an
 earlier call's partials: Q8_0 at 4096 rows (m = 512 with two splits, the
-others with more), Q4_K at 4096 rows (m = 128 with two splits, 16 with four),
+others with more), Q4_K at 1024 rows (m = 64, then 16),
 Q4_0 at 4096 rows (m = 300, then 20 in 32-row tiles), Q5_K at 4096 rows (m =
-64, then 16) and Q6_K at 1024 (m = 37, then 5); Q4_K at 14336 rows, which does
-not split, too.
+64, then 16) and Q6_K at 1024 rows of 8192 (m = 37, then 5); shapes that do not
+split (Q4_K at 14336 rows, Q6_K with K = 2048) too.
 """
 import ctypes
 
@@ -27,11 +27,12 @@ pytestmark = pytest.mark.gpu
 GEMM_TOL = 1e-2
 
 
-SPLIT = [(syn.Q8_0, 4096, 4096, (512, 200, 48)), (syn.Q4_K, 4096, 4096, (128, 16)), (syn.Q4_0, 4096, 4096, (300, 20)),
-         (syn.Q5_K, 4096, 4096, (64, 16)), (syn.Q6_K, 1024, 2048, (37, 5))]
+SPLIT = [(syn.Q8_0, 4096, 4096, (512, 200, 48)), (syn.Q4_K, 1024, 4096, (64, 16)), (syn.Q4_0, 4096, 4096, (300, 20)),
+         (syn.Q5_K, 4096, 4096, (64, 16)), (syn.Q6_K, 1024, 8192, (37, 5))]
 
 
-@pytest.mark.parametrize("type_id,rows,cols,ms", SPLIT + [(syn.Q4_K, 14336, 4096, (128, 16))])
+@pytest.mark.parametrize("type_id,rows,cols,ms", SPLIT + [(syn.Q4_K, 14336, 4096, (128, 16)),
+                                                          (syn.Q6_K, 1024, 2048, (37, 5))])
 def test_noalloc_gemm_matches_allocating_entry_point(type_id, rows, cols, ms):
     import torch
 
