@@ -787,6 +787,15 @@ int32_t gollek_hip_gemm_bf16(gollek_hip_weight *w, const uint16_t *x, int64_t x_
     return GOLLEK_HIP_OK;
 }
 
+// Split-K workspace of a device call.  The column kernel's calls (M <= 4) take
+// none, and asking for the plan of another kernel costs the host 0.1 to 0.3 us of
+// their 3 us.
+static size_t gemm_call_workspace(const gollek_hip_weight *w, const uint16_t *x, int64_t m) {
+    const uint8_t *const data = w->data != nullptr ? w->data : w->prep;
+    if (gollek::gemm_col_supported(w->type_id, w->row_bytes, (int)m, (int)w->rows, (int)w->cols, data, x)) return 0;
+    return gollek::gemm_workspace_bytes(w->type_id, (int)m, (int)w->rows, (int)w->cols);
+}
+
 int32_t gollek_hip_gemm_bf16_device(gollek_hip_weight *w, const uint16_t *x, int64_t m, float *y,
                                     void *stream, char *err, size_t err_len) {
     const int32_t rc = check_gemm(w, x, y, m, true, err, err_len);
@@ -795,7 +804,7 @@ int32_t gollek_hip_gemm_bf16_device(gollek_hip_weight *w, const uint16_t *x, int
     // for the largest split any m of this weight uses (below 16 MiB on 256
     // CUs), and kept until the handle is freed, so a launch in flight never
     // loses it.
-    const size_t need = gollek::gemm_workspace_bytes(w->type_id, (int)m, (int)w->rows, (int)w->cols);
+    const size_t need = gemm_call_workspace(w, x, m);
     if (need > 0) {
         std::lock_guard<std::mutex> lock(w->mu);
         if (w->gemm_ws == nullptr) {
@@ -829,7 +838,7 @@ int32_t gollek_hip_gemm_bf16_device_noalloc(gollek_hip_weight *w, const uint16_t
     // clearing; overlapping calls race).  A shape whose splits would need more
     // than the scratch holds is split less (the launcher picks the splits
     // that fit), down to none.
-    const size_t need = gollek::gemm_workspace_bytes(w->type_id, (int)m, (int)w->rows, (int)w->cols);
+    const size_t need = gemm_call_workspace(w, x, m);
     float *ws = nullptr;
     if (need > 0) {
         ws = (w->device >= 0 && w->device < kMaxDevices) ? g_scratch_ptr[w->device].load() : nullptr;
