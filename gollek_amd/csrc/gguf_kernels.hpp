@@ -198,12 +198,13 @@ hipError_t launch_moe_q40_mfma(const uint8_t *gate, const uint8_t *up, const uin
 
 // K-quant experts, many routes each, as grouped GEMMs (gguf_moe_gemm.hip):
 // gate / up of one K-quant type, down of any, hidden and inter multiples of
-// 256, weights 2-byte and x 16-byte aligned.
+// 256, weights 2-byte and x 16-byte aligned.  keep_wide: rows of x and h with
+// infinities or outliers of 2^20 are computed in fp32 (gguf_kq_f16.hpp).
 bool moe_gemm_supported(int gate_type, int up_type, int down_type, int E, int H, int I, int T, int top_k,
                         const uint8_t *gate, const uint8_t *up, const uint8_t *down, const float *x);
 hipError_t launch_moe_gemm(int gate_type, int down_type, const uint8_t *gate, const uint8_t *up, const uint8_t *down,
                            int E, int H, int I, const float *x, const int32_t *ids, const float *wts, int T,
-                           int top_k, float *out, uint8_t *ws, hipStream_t stream);
+                           int top_k, bool keep_wide, float *out, uint8_t *ws, hipStream_t stream);
 
 // Pieces of the MoE pipeline shared by its implementations (gguf_moe.hip,
 // gguf_moe_mfma.hip, gguf_moe_gemm.hip): routing (meta layout of moe_layout)

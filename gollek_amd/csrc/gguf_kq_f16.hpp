@@ -13,8 +13,8 @@
 // x: each (row, superblock) is scaled by a power of two that brings its
 // largest magnitude to [2^14, 2^15); bf16 elements are then exact in fp16
 // unless they are below 2^-31 of that maximum, where the error is at most 2^-39
-// of it.  Rows with an outlier of 2^20 times some 16 columns' largest and more
-// (kq_wide), and those with an infinity (the parts of a Q6_K product would cancel
+// of it.  Rows with an outlier of 2^20 times half the superblock's columns and
+// more (kq_wide), and those with an infinity (the parts of a Q6_K product would cancel
 // to NaN), are computed again by kq_wide_rows (Q4_K M = 512, 14336 x 4096: 229 us
 // with one such row, 1030 with 512 of them, 104 with none on the same card).
 //
@@ -273,12 +273,15 @@ __device__ __forceinline__ void kq_row_scale(float mx, float &s, float &inv) {
     inv = __uint_as_float(e - (14u << 23));
 }
 
-// Whether a row's superblock of maximum `mx` is one for kq_wide_rows, by 16 of
-// its columns, of maximum `lane_mx`: an infinity, or 16 that are not all zero
-// and below 2^-6 when scaled, where fp16's rounding is 2^-19 of their largest (an
-// outlier of 2^20 times the rest, its weights 0: 1.5e-7 of error in the result,
-// fp32 sums of K = 2048 1 to 6e-7).  The lanes that find it so (a ballot each: of
-// the two together it takes a select and a second comparison).
+// Whether a row's superblock of maximum `mx` is one for kq_wide_rows: an
+// infinity, or kWideRuns of its 16 runs of 16 columns each of a maximum
+// (`lane_mx`) that is not 0 and below 2^-6 when scaled, where fp16's rounding is
+// 2^-19 of it (an outlier of 2^20 times the rest, its weights 0: 1.5e-7 of error in
+// the result, fp32 sums of K = 2048 1 to 6e-7).  Fewer such runs are no outlier's
+// superblock but the tails of a gated activation beside values that outweigh
+// them by 2^20.  The lanes that find one (a ballot each: of the two together it
+// takes a select and a second comparison); an infinity counts in all 16.
+constexpr int kWideRuns = 8;
 __device__ __forceinline__ uint64_t kq_wide(float lane_mx, float mx, float inv) {
     return __builtin_amdgcn_ballot_w64(__float_as_uint(lane_mx) - 1u < __float_as_uint(inv) - (6u << 23)) |
            __builtin_amdgcn_ballot_w64(mx == __builtin_inff());

@@ -36,7 +36,7 @@ struct XRows {
         x[1] = *reinterpret_cast<const v4u *>(p + 8);
     }
     // p0, p1: the lane's two pieces, mins: its sub-block's half of a min piece;
-    // returns the lanes that find their row a wide one
+    // returns the lanes that find their row a wide one, if enough of them do
     __device__ __forceinline__ uint64_t store(uint8_t *p0, uint8_t *p1, uint8_t *mins, float *scale, int lane) const {
         float v[16], mx = 0.0f;
 #pragma unroll
@@ -67,7 +67,8 @@ struct XRows {
             *reinterpret_cast<uint2 *>(mins) = kq_min_digits(t);  // both lanes write the same 8 bytes
         }
         if ((lane & 15) == 0) *scale = inv;
-        return kq_wide(lane_mx, mx, inv);
+        const uint64_t found = kq_wide(lane_mx, mx, inv);
+        return __builtin_popcountll(found) >= kWideRuns ? found : 0u;  // (of the four rows together)
     }
 };
 

@@ -882,12 +882,18 @@ hipError_t launch_moe_generic(int gate_type, int up_type, int down_type, const u
 // equal; Q5_K, 96 equal; eight experts 56 routes 39 / 41), and with Q5_K down rows it is the faster one up to five
 // routes per expert (128 x 1536, hidden 2048: three 1.34 times as fast, four 1.16,
 // five 0.95; with hidden 1024, x 512, the grouped GEMM from three: 0.78).
+// Top-k of at most 4 k experts is mostly one device's share of a larger layer,
+// whose routes are other devices' but for a part that only the device knows:
+// with an eighth of 128 routes valid (16 of 128 experts x 768, hidden 2048, Q4_K,
+// 16 tokens) 21 us on the two-launch passes, 35 here; with all of them valid 58 /
+// 46.  From 160 routes the gain if all are is the larger one.
 static bool moe_gemm_chosen(bool tile_passes, int down_type, int E, int H, int I, int T, int top_k) {
     const int64_t P = (int64_t)T * top_k;
     if (!tile_passes) return P >= E && (T > 2 || P >= 2 * (int64_t)E);
     const bool expert_major = moe_kq_expert_major_down(down_type, E, H, I, T, top_k), q5 = down_type == kQ5_K;
     const int64_t per_expert = expert_major && q5 && H >= 2048 ? 5 : 3;
-    const int64_t least = !expert_major ? 56 : E > 4 ? 64 : q5 ? 96 : 80;
+    const bool share = top_k >= 4 && 4 * top_k >= E;
+    const int64_t least = share ? 160 : !expert_major ? 56 : E > 4 ? 64 : q5 ? 96 : 80;
     return P >= per_expert * E && P >= least;
 }
 
@@ -924,7 +930,8 @@ hipError_t launch_moe(int gate_type, int up_type, int down_type, const uint8_t *
                              moe_kq_mfma_supported(gate_type, down_type, E, H, I, T, top_k, x);
     if (tuning().moe_variant != 1 && moe_gemm_chosen(tile_passes, down_type, E, H, I, T, top_k) &&
         moe_gemm_supported(gate_type, up_type, down_type, E, H, I, T, top_k, gate, up, down, x))
-        return launch_moe_gemm(gate_type, down_type, gate, up, down, E, H, I, x, ids, wts, T, top_k, out, ws, stream);
+        return launch_moe_gemm(gate_type, down_type, gate, up, down, E, H, I, x, ids, wts, T, top_k, !tile_passes, out, ws,
+                               stream);
     if (tile_passes)
         return launch_moe_kq_mfma(gate_type, down_type, gate, up, down, E, H, I, x, ids, wts, T, top_k, out, ws,
                                   stream);

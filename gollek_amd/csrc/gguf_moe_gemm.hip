@@ -17,7 +17,10 @@
 // the workspace's ypair region (free until the down pass), h's in place.
 // Superblocks of too wide a range and those with an infinity (kq_wide) stay
 // fp32, marked by a negative scale, and the rows that hold one are computed
-// again from the packed weights.
+// again from the packed weights -- on the shapes that only the fp32 row kernels
+// take otherwise.  Where the two-launch passes do, x and h were digits of 22 bits
+// already, and h may well be of that kind (gates far below 0: e^-|g| over many
+// powers of two; 256 tokens of random weights 154 us without, 187 with).
 //
 // What bounds it: a workgroup's stage is short (34 MFMAs a wave at one row
 // tile), so its loads' latency shows; small tiles keep several workgroups on
@@ -53,7 +56,7 @@ namespace {
 // rec is its 256 floats and its scale negative (mins not written).  The lanes
 // have read their columns before they write (rec may be v itself).
 template <int T>
-__device__ __forceinline__ void record_row(const float *v, int64_t r, int sb, int K, uint8_t *rec,
+__device__ __forceinline__ void record_row(const float *v, int64_t r, int sb, int K, int keep_wide, uint8_t *rec,
                                            uint8_t *__restrict__ mins, float *__restrict__ scales) {
     const int n = (int)threadIdx.x & 15;
     const int64_t rs = r * (K / kQK) + sb;
@@ -70,7 +73,7 @@ __device__ __forceinline__ void record_row(const float *v, int64_t r, int sb, in
     kq_row_scale(mx, s, inv);
     uint8_t *const dst = rec + rs * 1024;
     const uint64_t found = kq_wide(lane_mx, mx, inv);
-    if (((found >> (threadIdx.x & 48u)) & 0xFFFFu) != 0u) {  // the row's 16 lanes alike
+    if (keep_wide && __popc((uint32_t)(found >> (threadIdx.x & 48u)) & 0xFFFFu) >= kWideRuns) {  // the row's lanes alike
 #pragma unroll
         for (int i = 0; i < 4; i++) reinterpret_cast<f32x4 *>(dst + 64 * n)[i] = x[i];
         if (n == 0) scales[rs] = -inv;
@@ -107,10 +110,10 @@ __device__ __forceinline__ void record_row(const float *v, int64_t r, int sb, in
 
 // Records of `rows` rows, 16 rows and a superblock a workgroup.
 template <int T>
-__global__ __launch_bounds__(256) void moe_records_kernel(const float *v, int rows, int K, uint8_t *rec,
+__global__ __launch_bounds__(256) void moe_records_kernel(const float *v, int rows, int K, int keep_wide, uint8_t *rec,
                                                           uint8_t *__restrict__ mins, float *__restrict__ scales) {
     const int r = 16 * (int)blockIdx.y + (int)(threadIdx.x >> 4);
-    if (r < rows) record_row<T>(v, r, (int)blockIdx.x, K, rec, mins, scales);  // whole rows of 16 lanes
+    if (r < rows) record_row<T>(v, r, (int)blockIdx.x, K, keep_wide, rec, mins, scales);  // whole rows of 16 lanes
 }
 
 // The first launch: workgroup 0 routes, the others build x's records (64 rows'
@@ -121,7 +124,8 @@ __global__ __launch_bounds__(kRouteThreads) void moe_front_kernel(const int32_t 
                                                                   int group, int chunks, int keys_in_lds,
                                                                   int32_t *__restrict__ meta,
                                                                   int2 *__restrict__ items, const float *x, int rows,
-                                                                  int K, uint8_t *rec, uint8_t *__restrict__ mins,
+                                                                  int K, int keep_wide, uint8_t *rec,
+                                                                  uint8_t *__restrict__ mins,
                                                                   float *__restrict__ scales) {
     extern __shared__ int32_t sh[];
     if (blockIdx.x == 0) {
@@ -130,7 +134,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_front_kernel(const int32_t 
     }
     const int nsb = K / kQK;
     const int64_t i = (int64_t)(blockIdx.x - 1) * (kRouteThreads / 16) + (int)(threadIdx.x >> 4);
-    if (i < (int64_t)rows * nsb) record_row<T>(x, i / nsb, (int)(i % nsb), K, rec, mins, scales);
+    if (i < (int64_t)rows * nsb) record_row<T>(x, i / nsb, (int)(i % nsb), K, keep_wide, rec, mins, scales);
 }
 
 namespace {
@@ -373,13 +377,15 @@ hipError_t launch_pass_type(int type, A... a) {
     return launch_pass<kQ6_K, GATED>(a...);
 }
 
-hipError_t launch_records(int type, const float *v, int64_t rows, int K, uint8_t *rec, uint8_t *mins, float *scales,
-                          hipStream_t stream) {
+hipError_t launch_records(int type, const float *v, int64_t rows, int K, bool keep_wide, uint8_t *rec, uint8_t *mins,
+                          float *scales, hipStream_t stream) {
     const dim3 grid((unsigned)(K / kQK), (unsigned)((rows + 15) / 16));
     if (type == kQ6_K)
-        hipLaunchKernelGGL(moe_records_kernel<kQ6_K>, grid, dim3(256), 0, stream, v, (int)rows, K, rec, mins, scales);
+        hipLaunchKernelGGL(moe_records_kernel<kQ6_K>, grid, dim3(256), 0, stream, v, (int)rows, K,
+                           (int)keep_wide, rec, mins, scales);
     else
-        hipLaunchKernelGGL(moe_records_kernel<kQ4_K>, grid, dim3(256), 0, stream, v, (int)rows, K, rec, mins, scales);
+        hipLaunchKernelGGL(moe_records_kernel<kQ4_K>, grid, dim3(256), 0, stream, v, (int)rows, K,
+                           (int)keep_wide, rec, mins, scales);
     return hipGetLastError();
 }
 
@@ -406,7 +412,7 @@ bool moe_gemm_supported(int gate_type, int up_type, int down_type, int E, int H,
 
 hipError_t launch_moe_gemm(int gate_type, int down_type, const uint8_t *gate, const uint8_t *up, const uint8_t *down,
                            int E, int H, int I, const float *x, const int32_t *ids, const float *wts, int T,
-                           int top_k, float *out, uint8_t *ws, hipStream_t stream) {
+                           int top_k, bool keep_wide, float *out, uint8_t *ws, hipStream_t stream) {
     const MoeLayout L = moe_layout(T, top_k, H, I, E);
     const int P = T * top_k, mt = item_tiles(P, E);
     int32_t *meta = reinterpret_cast<int32_t *>(ws + L.meta);
@@ -421,7 +427,7 @@ hipError_t launch_moe_gemm(int gate_type, int down_type, const uint8_t *gate, co
     const dim3 fgrid((unsigned)(1 + (xrows + kRouteThreads / 16 - 1) / (kRouteThreads / 16)));
     auto front = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, fgrid, dim3(kRouteThreads), rp.lds_bytes, stream, ids, wts, P, E, 16 * mt,
-                           rp.chunks, rp.keys_in_lds, meta, list, x, T, H, xrec, ws + xt.mins,
+                           rp.chunks, rp.keys_in_lds, meta, list, x, T, H, (int)keep_wide, xrec, ws + xt.mins,
                            reinterpret_cast<float *>(ws + xt.scales));
     };
     gate_type == kQ6_K ? front(&moe_front_kernel<kQ6_K>) : front(&moe_front_kernel<kQ4_K>);
@@ -431,7 +437,7 @@ hipError_t launch_moe_gemm(int gate_type, int down_type, const uint8_t *gate, co
                                reinterpret_cast<const float *>(ws + xt.scales), top_k, list, nitems, offsets, pairs, h,
                                stream);
     if (e != hipSuccess) return e;
-    e = launch_records(down_type, h, P, I, hrec, ws + ht.mins, reinterpret_cast<float *>(ws + ht.scales), stream);
+    e = launch_records(down_type, h, P, I, keep_wide, hrec, ws + ht.mins, reinterpret_cast<float *>(ws + ht.scales), stream);
     if (e != hipSuccess) return e;
     e = launch_pass_type<false>(down_type, mt, (int64_t)P, E, items, down, down, H, I, hrec, ws + ht.mins,
                                 reinterpret_cast<const float *>(ws + ht.scales), 1, list, nitems, offsets, pairs,
