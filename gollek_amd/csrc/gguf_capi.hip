@@ -117,7 +117,7 @@ int g_initialised_device = -1;
 // process ends.  On the host, `scratch` only names that array; kernels get
 // the per-device address hipGetSymbolAddress returns, resolved once per
 // device (with the device current) when the library first sets it up.
-constexpr size_t kGemmScratchBytes = (size_t)16 << 20;  // gemm_workspace_bytes < 16 MiB on 256 CUs
+constexpr size_t kGemmScratchBytes = (size_t)16 << 20;  // gemm_workspace_bytes <= 16 MiB on 256 CUs
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) float scratch[kGemmScratchBytes / sizeof(float)];
 std::atomic<float *> g_scratch_ptr[kMaxDevices];
@@ -801,7 +801,7 @@ int32_t gollek_hip_gemm_bf16_device(gollek_hip_weight *w, const uint16_t *x, int
     const int32_t rc = check_gemm(w, x, y, m, true, err, err_len);
     if (rc != GOLLEK_HIP_OK) return rc;
     // The handle's split-K workspace: allocated at the first call that splits,
-    // for the largest split any m of this weight uses (below 16 MiB on 256
+    // for the largest split any m of this weight uses (16 MiB at most on 256
     // CUs), and kept until the handle is freed, so a launch in flight never
     // loses it.
     const size_t need = gemm_call_workspace(w, x, m);

@@ -503,17 +503,18 @@ __global__ __launch_bounds__(256) void gemm_tile_reduce_kernel(const float *__re
 
 namespace {
 
-// Row tiles of X per workgroup.  Shapes that may split K (whole 256-column
-// rounds): the smallest of 1, 2, 4, 8 that covers M, so that small M computes
-// no padding rows.  Q8_0 up to M = 128 with so few column tiles that 128-row
-// tiles would split K eight ways takes 64-row tiles split four ways instead:
-// three partial tiles per output in place of seven (M = 128, N = 4096: 18.7
-// against 19.7 us; the Q4_0 tiles at N = 14336 measured slower with 64 rows).
-// Other K run unsplit (they always have: see gemm_may_split): the tile height with the shortest rounds over the CUs
-// (a stage of 1, 2, 4 or 8 row tiles takes about 0.46, 0.54, 0.69 and 0.95 us,
-// a tile's start and end 3 us).  N = 5760, K = 2880, M = 100: 20.6 us, 40.9 on the
-// converted-copy kernel these shapes took before; K = 2912, M = 256, N = 4000:
-// 23 us, 1220 with one thread per output.
+// Row tiles of X per workgroup.  K a multiple of 256: the smallest of 1, 2, 4, 8
+// that covers M, so that small M computes no padding rows (where K is one of 512
+// too, such tiles may split K; an odd multiple of 256, 2816 or 11008, neither
+// splits nor takes the heights below).  Q8_0 up to M = 128 with so few column
+// tiles that 128-row tiles would split K eight ways takes 64-row tiles split four
+// ways instead: three partial tiles per output in place of seven (M = 128, N =
+// 4096: 18.7 against 19.7 us; the Q4_0 tiles at N = 14336 measured slower with 64
+// rows).  Other K run unsplit (they always have: see gemm_may_split): the tile
+// height with the shortest rounds over the CUs (a stage of 1, 2, 4 or 8 row tiles
+// takes about 0.46, 0.54, 0.69 and 0.95 us, a tile's start and end 3 us).  N =
+// 5760, K = 2880, M = 100: 20.2 us, 40.9 on the converted-copy kernel these shapes
+// took before; K = 2912, M = 256, N = 4000: 23 us, 1220 with one thread per output.
 int tile_mt(int type_id, int M, int N, int K) {
     if (K % 256 != 0) {
         constexpr float kStage[4] = {0.46f, 0.54f, 0.69f, 0.95f};

@@ -2,19 +2,20 @@
 // fp16 matrix cores (gguf_kq_f16.hpp), X bf16 (row-major M x K), fp32
 // accumulate; semantics as gguf_gemm_tile.hip (Q4_K: RT/GgufQ4RawDot.java:331-674).
 //
-// What bounds it: above M ~ 256 the VALU instructions beside the MFMAs.  A
-// wave's 32 columns of a superblock take 18 MFMAs per row tile (16 cycles
-// each) and, at 128 rows, per MFMA 1.6 instructions to widen the codes, 2.1 to
-// scale and convert x and 1.3 to apply d, min and the row scale; timing copies
-// without the x conversion ran Q4_K M = 2048, 14336 x 4096 in 270 us, without
-// the MFMAs in 273 us, whole 345 us.  Below that the latency of a stage (the
+// What bounds it: above M ~ 256 MFMA and VALU issue, whose phases in a
+// workgroup's waves hardly overlap (Q4_K M = 512: 0.27 and 0.40 of the time).  A
+// wave's 32 columns of a superblock take 18 MFMAs per row tile (16 cycles each)
+// and, at 128 rows, per MFMA 5.6 VALU instructions: 1.6 to widen the codes, 2.3 to
+// scale and convert x, 0.9 to apply d, min and the row scale; timing copies of an
+// earlier form (345 us at Q4_K M = 2048, 14336 x 4096) ran in 270 without the x
+// conversion, in 273 without the MFMAs.  Below that the latency of a stage (the
 // next superblock's bytes are requested late in it), so small M takes small
 // tiles with the superblocks spread over the waves.
 // Against the bf16 kernel with one FMA per 32 columns and output that this
-// replaces: Q4_K M = 2048 456 -> 345 us (697 TFLOP/s), M = 512 134 -> 97;
-// Q6_K M = 333, 4096 x 14336 183 -> 100 us (its scale groups of 16 took three
-// half-empty MFMAs); Q4_K M = 16 19.5 -> 13.9 us (14.9 with the first raw bytes
-// of W requested only once the first x stood in LDS).
+// replaces: Q4_K M = 2048 463 -> 341 us (705 TFLOP/s), M = 512 134 -> 89; Q6_K M =
+// 333, 4096 x 14336 181 -> 99 us (its scale groups of 16 took three half-empty
+// MFMAs); Q4_K M = 16 19.3 -> 15.1 us a layer of four (the first raw bytes of W
+// requested only once the first x stood in LDS: 1 us more).
 #include "gguf_gemm_plan.hpp"
 #include "gguf_kq_f16.hpp"
 

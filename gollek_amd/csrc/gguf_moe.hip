@@ -879,9 +879,10 @@ hipError_t launch_moe_generic(int gate_type, int up_type, int down_type, const u
 // 3 routes: 102 / 77 us; 8 x 1536, 32 routes in all: 38 / 46 us, 64 routes: 50 /
 // 46).  Their expert-major down pass holds longer: few experts give the grouped
 // GEMM few workgroups (one of 1536, hidden 2048: Q4_K, 64 routes 46 / 56 us, 80
-// equal; Q5_K, 96 equal; eight experts 56 routes 39 / 41), and with Q5_K down rows it is the faster one up to five
-// routes per expert (128 x 1536, hidden 2048: three 1.34 times as fast, four 1.16,
-// five 0.95; with hidden 1024, x 512, the grouped GEMM from three: 0.78).
+// equal; Q5_K, 96 equal; eight experts 56 routes 39 / 41), and with Q5_K down rows
+// it is the faster one up to five routes per expert (128 x 1536, hidden 2048: three
+// 1.34 times as fast, four 1.16, five 0.95; with hidden 1024, x 512, the grouped
+// GEMM from three: 0.78).
 // Top-k of at most 4 k experts is mostly one device's share of a larger layer,
 // whose routes are other devices' but for a part that only the device knows:
 // with an eighth of 128 routes valid (16 of 128 experts x 768, hidden 2048, Q4_K,

@@ -11,8 +11,8 @@
 // maximum in [2^14, 2^15), v = hi + lo leaves an error below 2^-23 of v or 2^-39
 // of the maximum (the two-launch passes keep 2^-22 of it; against the fp32 row
 // kernels the roundings of the products weigh more: 4.5e-7 of error against
-// 7e-7); both digits
-// contract against the same exact weight operand into one fp32 accumulator.
+// 7e-7); both digits contract against the same exact weight operand into one
+// fp32 accumulator.
 // They are built once per vector ("records") by a kernel of its own, x's into
 // the workspace's ypair region (free until the down pass), h's in place.
 // Superblocks of too wide a range and those with an infinity (kq_wide) stay
@@ -25,9 +25,9 @@
 // What bounds it: a workgroup's stage is short (34 MFMAs a wave at one row
 // tile), so its loads' latency shows; small tiles keep several workgroups on
 // a CU.  128 experts x 768, hidden 2048, Q4_K gate / up, Q6_K down, 256 tokens x
-// top-8: 717 us on the passes of gguf_moe_mfma.hip, 184 here (the launches beside
-// the two GEMMs 24 us; the weights are 391 MB); 32 x 1280,
-// hidden 2816, 256 tokens x top-4: 2435 us on the row kernels, 157 here.
+// top-8: 714 us on the passes of gguf_moe_mfma.hip, 176 here (the launches beside
+// the two GEMMs 25 us; the weights are 391 MB); 32 x 1280, hidden 2816, 100 tokens
+// x top-4: 918 us on the row kernels, 109 here.
 //
 // Launches: routing (a list of (expert, first route) items of at most 16 MT
 // routes) with x's records, gate/up (h), h records, down (a row per route), combine
