@@ -884,17 +884,19 @@ hipError_t launch_moe_generic(int gate_type, int up_type, int down_type, const u
 // 1.34 times as fast, four 1.16, five 0.95; with hidden 1024, x 512, the grouped
 // GEMM from three: 0.78).
 // Top-k of at most 4 k experts is mostly one device's share of a larger layer,
-// whose routes are other devices' but for a part that only the device knows:
-// with an eighth of 128 routes valid (16 of 128 experts x 768, hidden 2048, Q4_K,
-// 16 tokens) 21 us on the two-launch passes, 35 here; with all of them valid 58 /
-// 46.  From 160 routes the gain if all are is the larger one.
+// whose routes are other devices' but for a part that only the device knows, of
+// at most 2 k experts nothing else.  Of 16 experts x 768, hidden 2048, Q4_K with
+// Q6_K down, top-8: an eighth of the routes valid, 160 routes 30 / 39 us, 256 33 /
+// 40, 320 40 / 41, 400 49 / 42; all of them valid, 160 routes 73 / 41.  So the
+// lines are 320 routes up to 2 k experts, and 160 up to 4 k (32 experts, top-8, 160
+// routes: an eighth valid 32 / 45, all 74 / 52).
 static bool moe_gemm_chosen(bool tile_passes, int down_type, int E, int H, int I, int T, int top_k) {
     const int64_t P = (int64_t)T * top_k;
     if (!tile_passes) return P >= E && (T > 2 || P >= 2 * (int64_t)E);
     const bool expert_major = moe_kq_expert_major_down(down_type, E, H, I, T, top_k), q5 = down_type == kQ5_K;
     const int64_t per_expert = expert_major && q5 && H >= 2048 ? 5 : 3;
     const bool share = top_k >= 4 && 4 * top_k >= E;
-    const int64_t least = share ? 160 : !expert_major ? 56 : E > 4 ? 64 : q5 ? 96 : 80;
+    const int64_t least = share ? (2 * top_k >= E ? 320 : 160) : !expert_major ? 56 : E > 4 ? 64 : q5 ? 96 : 80;
     return P >= per_expert * E && P >= least;
 }
 

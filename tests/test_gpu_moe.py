@@ -344,6 +344,24 @@ def test_moe_single_routes_take_the_row_kernels(gt, dt, E, H, I, T, k, moe_varia
         t.close()
 
 
+# A device's share of a layer's experts (an eighth of the routes valid): 256 routes
+# stay on the two-launch passes, which compute a token's routes for themselves,
+# so pieces of 6 tokens (48 routes, always theirs) give the same bits.
+@pytest.mark.parametrize("gt,dt", [(syn.Q4_K, syn.Q4_K), (syn.Q5_K, syn.Q6_K), (syn.Q6_K, syn.Q6_K)])
+def test_moe_share_of_experts_takes_the_passes(gt, dt):
+    print(f"[gpu] moe share gate={gt} down={dt}", flush=True)
+    E, H, I, T, k = 16, 512, 256, 32, 8
+    *_, tg, tu, td = _experts(E, H, I, seed=E + gt, down_type=dt, gate_type=gt)
+    ids, w = syn.moe_routing(T, 8 * E, k, seed=83)
+    ids = np.where(ids < E, ids, -1).astype(np.int32)
+    x = syn.activation(T * H, seed=84).reshape(T, H)
+    out = ops.moe_grouped(tg, tu, td, E, x, ids, w)
+    parts = [ops.moe_grouped(tg, tu, td, E, x[t:t + 6], ids[t:t + 6], w[t:t + 6]) for t in range(0, T, 6)]
+    np.testing.assert_array_equal(out, np.concatenate(parts))
+    for t in (tg, tu, td):
+        t.close()
+
+
 @pytest.mark.parametrize("gt,dt", [(syn.Q4_0, syn.Q4_0), (syn.Q5_K, syn.Q6_K), (syn.Q5_K, syn.Q5_K),
                                    (syn.Q6_K, syn.Q6_K)])
 def test_moe_matrix_core_equals_row_kernels(gt, dt, moe_variant):
