@@ -402,13 +402,20 @@ __device__ __forceinline__ void kq_stages(f32x4 (&acc)[MT][2], const uint8_t *co
                 __builtin_amdgcn_sched_barrier(0);
             });
         });
+        int eg = g, en = n;
+        if constexpr (T == kQ4_K && MT == 8) {  // no registers for offsets that are kept through the stage
+            int l = lane;
+            asm volatile("" : "+v"(l));
+            eg = l >> 4;
+            en = l & 15;
+        }
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
             const uint8_t *const unit = cur + mt * U::kBytes;
-            const f32x4 inv = *reinterpret_cast<const f32x4 *>(unit + U::kScales + 16 * g);
+            const f32x4 inv = *reinterpret_cast<const f32x4 *>(unit + U::kScales + 16 * eg);
             f32x4 pm[2], ps[2];
             if constexpr (Op::kMins) {
-                const f16x8 am = *reinterpret_cast<const f16x8 *>(unit + U::kMins + 64 * n + 16 * g);
+                const f16x8 am = *reinterpret_cast<const f16x8 *>(unit + U::kMins + 64 * en + 16 * eg);
 #pragma unroll
                 for (int nt = 0; nt < 2; nt++) {
                     pm[nt] = mfma_f16(am, op[nt].bm, zero);

@@ -12,10 +12,11 @@
 // next superblock's bytes are requested late in it), so small M takes small
 // tiles with the superblocks spread over the waves.
 // Against the bf16 kernel with one FMA per 32 columns and output that this
-// replaces: Q4_K M = 2048 463 -> 341 us (705 TFLOP/s), M = 512 134 -> 89; Q6_K M =
+// replaces: Q4_K M = 2048 463 -> 341 us (705 TFLOP/s), M = 512 134 -> 85; Q6_K M =
 // 333, 4096 x 14336 181 -> 99 us (its scale groups of 16 took three half-empty
 // MFMAs); Q4_K M = 16 19.3 -> 15.1 us a layer of four (the first raw bytes of W
 // requested only once the first x stood in LDS: 1 us more).
+#include "gguf_dot4.hpp"
 #include "gguf_gemm_plan.hpp"
 #include "gguf_kq_f16.hpp"
 
@@ -35,6 +36,10 @@ struct XRows {
     __device__ __forceinline__ void load(const uint16_t *p) {
         x[0] = *reinterpret_cast<const v4u *>(p);
         x[1] = *reinterpret_cast<const v4u *>(p + 8);
+    }
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+        x[0] = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
+        x[1] = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 16, 0);
     }
     // p0, p1: the lane's two pieces, mins: its sub-block's half of a min piece;
     // returns the lanes that find their row a wide one, if enough of them do
@@ -129,11 +134,29 @@ __global__ __launch_bounds__(64 * NW *KW, MT == 1 && NW == 2 ? 4 : 1) void gemm_
     kq_place<T>(n, xg, xk0, xk1);
     XRows<T> xr[2];
     uint64_t found[kPer] = {};
+    // Q4_K's 128-row tile has no registers for four row pointers (they and the
+    // epilogue's LDS offsets, spilled, were waited for with W's bytes behind them: M =
+    // 512, 14336 x 4096, 89.2 against 84.7 us): it reads its rows of X through a
+    // descriptor, one lane offset and a wave's, kept out of the loop's carried
+    // registers; rows past M read as zeros.  Q5_K's measured 1 % slower so, Q6_K's
+    // 1.2 times (it spills inside the loop).
+    constexpr bool kDescriptor = T == kQ4_K && MT == 8;
+    const __amdgpu_buffer_rsrc_t xs =
+        wave_buffer(reinterpret_cast<const uint8_t *>(X + (int64_t)m0 * K),
+                    kDescriptor ? 2u * (uint32_t)(M - m0 < kTileM ? M - m0 : kTileM) * (uint32_t)K : 0u);
+    const uint32_t xo = 2u * ((uint32_t)g * (uint32_t)K + 16u * (uint32_t)n);
     auto load_x = [&](XRows<T> &to, int j, int st) {
         const int q = wave + kWaves * j, u = q >> 2, sb = st * KW + u / MT;
-        const int r = m0 + 16 * (u % MT) + 4 * (q & 3) + g;
-        // (rows past M repeat row M - 1; their results are not stored)
-        to.load(X + (int64_t)(r < M ? r : M - 1) * K + (int64_t)(sb < nsb ? sb : nsb - 1) * kQK + 16 * n);
+        if constexpr (kDescriptor) {
+            uint32_t at = 2u * ((uint32_t)(16 * (u % MT) + 4 * (q & 3)) * (uint32_t)K +
+                                (uint32_t)((sb < nsb ? sb : nsb - 1) * kQK));
+            asm volatile("" : "+s"(at));
+            to.load(xs, xo + at);
+        } else {
+            const int r = m0 + 16 * (u % MT) + 4 * (q & 3) + g;
+            // (rows past M repeat row M - 1; their results are not stored)
+            to.load(X + (int64_t)(r < M ? r : M - 1) * K + (int64_t)(sb < nsb ? sb : nsb - 1) * kQK + 16 * n);
+        }
     };
     auto store_x = [&](const XRows<T> &from, int j, int b) {
         const int q = wave + kWaves * j, u = q >> 2, lr = 4 * (q & 3) + g;
@@ -230,7 +253,7 @@ constexpr GemmPlanCost kQ4KPlans[] = {
     {1, 1, 4, 2, 3.30f, 2.87f}, {1, 1, 8, 1, 2.70f, 3.17f}, {1, 2, 4, 1, 2.19f, 2.19f},
     {2, 2, 2, 2, 3.90f, 3.25f}, {2, 2, 4, 1, 2.98f, 3.31f}, {2, 4, 2, 1, 2.94f, 2.51f},
     {4, 4, 2, 1, 4.18f, 3.71f}, {4, 8, 1, 1, 3.77f, 2.96f}, {6, 8, 1, 1, 5.51f, 3.73f},
-    {8, 8, 1, 1, 6.48f, 5.01f}};
+    {8, 8, 1, 1, 6.48f, 4.90f}};
 constexpr GemmSplitCost kQ4KSplit = {2.88f, 0.179f};
 constexpr GemmPlanCost kQ5KPlans[] = {
     {1, 1, 4, 2, 3.49f, 3.74f}, {1, 1, 8, 1, 2.65f, 4.14f}, {1, 2, 4, 1, 2.23f, 3.24f},
@@ -280,7 +303,9 @@ bool launch_plan(const GemmPlan &p, A... a) {
 }  // namespace
 
 bool kq_gemm_supported(int type_id, int64_t row_bytes, int N, int K, const void *w, const void *x) {
+    // (Q4_K: 128 rows of X lie within the 2^31 bytes of a buffer descriptor)
     return (type_id == kQ4_K || type_id == kQ5_K || type_id == kQ6_K) && K > 0 && K % kQK == 0 && N > 0 &&
+           (type_id != kQ4_K || K < 1 << 23) &&
            ((reinterpret_cast<uintptr_t>(w) | (uintptr_t)row_bytes) & 1u) == 0 &&
            (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
 }
