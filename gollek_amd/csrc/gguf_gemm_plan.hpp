@@ -3,9 +3,12 @@
 //
 // A tile is 16 mt rows of X by 32 nw rows of W on nw * kw waves, its stages kw
 // chunks of 256 columns.  The time of a launch is modelled as the rounds of
-// workgroups over the CUs (half of it by whole rounds, half by the mean, since
-// a last round that is nearly empty runs faster) times a tile's start and end
-// and its stages, plus, for K cut into S parts, the reduction launch.  The
+// workgroups over the CUs (of the 256-column tiles by whole rounds, of the others
+// half of it and half by the mean, since there a last round that is nearly empty
+// runs faster) times a tile's start and end and its stages, plus, for K cut into S
+// parts, the reduction launch.  (256 columns, Q4_K, N = 11008, K = 4096: 1.34 rounds
+// of 64 rows 100 us, one round of 128 rows 85; 3.02 rounds of 96 rows at M = 1672
+// 264, 2.35 of 128 254.)  The
 // constants are fitted to all plans' times over M = 5 .. 2048 and twelve N x K
 // (177 shapes a type): the plan picked is within 1 % of the fastest on average,
 // one shape of a type at most 19 to 44 %.
@@ -52,7 +55,7 @@ GemmPlan pick_gemm_plan(const GemmPlanCost (&plans)[PLANS], GemmSplitCost split,
         for (int S = 1; S <= 8 && S <= stages && (S == 1 || (size_t)(S - 1) * mn <= ws_bytes); S++) {
             const double r = (double)tiles * S / (cus * p.per_cu);
             const double whole = (double)(long)(r + 0.999999);
-            const double rounds = 0.5 * whole + 0.5 * (r > 1.0 ? r : 1.0);
+            const double rounds = p.nw == 8 ? whole : 0.5 * whole + 0.5 * (r > 1.0 ? r : 1.0);
             double us = rounds * (p.tile_us + p.stage_us * ((stages + S - 1) / S));
             if (p.per_cu > 1 && (double)tiles * S <= cus) us *= kGemmAlone;
             if (S > 1) us += split.launch_us + split.mb_us * 2.0 * S * mn * 1e-6;
