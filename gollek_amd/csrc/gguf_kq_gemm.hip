@@ -3,7 +3,7 @@
 // accumulate; semantics as gguf_gemm_tile.hip (Q4_K: RT/GgufQ4RawDot.java:331-674).
 //
 // What bounds it: above M ~ 256 MFMA and VALU issue, whose phases in a
-// workgroup's waves hardly overlap (Q4_K M = 512: 0.27 and 0.40 of the time).  A
+// workgroup's waves hardly overlap (Q4_K M = 512: 0.29 and 0.42 of the time).  A
 // wave's 32 columns of a superblock take 18 MFMAs per row tile (16 cycles each)
 // and, at 128 rows, per MFMA 5.6 VALU instructions: 1.6 to widen the codes, 2.3 to
 // scale and convert x, 0.9 to apply d, min and the row scale; timing copies of an
@@ -12,7 +12,7 @@
 // next superblock's bytes are requested late in it), so small M takes small
 // tiles with the superblocks spread over the waves.
 // Against the bf16 kernel with one FMA per 32 columns and output that this
-// replaces: Q4_K M = 2048 463 -> 341 us (705 TFLOP/s), M = 512 134 -> 85; Q6_K M =
+// replaces: Q4_K M = 2048 463 -> 338 us (711 TFLOP/s), M = 512 134 -> 85; Q6_K M =
 // 333, 4096 x 14336 181 -> 99 us (its scale groups of 16 took three half-empty
 // MFMAs); Q4_K M = 16 19.3 -> 15.1 us a layer of four (the first raw bytes of W
 // requested only once the first x stood in LDS: 1 us more).
